@@ -41,7 +41,9 @@ enum senk_status {
     SENK_ERR_UNSUPPORTED = 9,    /* shape outside what the kernels support                     */
     SENK_ERR_SCHEDULE = 10,      /* a factor entry couples two blocks scheduled together       */
     SENK_ERR_TIMEOUT = 11,       /* a single-launch triangular solve gave up waiting on an
-                                    earlier level (the result of that solve is invalid)      */
+                                    earlier level (the result of that solve is invalid);
+                                    solves on caller arrays report it at the next driver end,
+                                    senk_ctx_synchronize or senk_memcpy_dtoh                 */
     SENK_ERR_IO = 12,            /* a file could not be opened or read                         */
     SENK_ERR_FORMAT = 13         /* a file is not a MatrixMarket matrix the reader supports    */
 };

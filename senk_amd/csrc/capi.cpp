@@ -65,6 +65,12 @@ static int arena_get(DevBuf &a, size_t bytes, void **out) {
     *out = a.p;
     return SENK_OK;
 }
+int ctx_sweep_check(Ctx *c) {
+    if (!c->sweep_err || !__atomic_load_n(c->sweep_err, __ATOMIC_ACQUIRE)) return SENK_OK;
+    __atomic_store_n(c->sweep_err, 0u, __ATOMIC_RELEASE);
+    record_error("a single-launch triangular solve gave up a wait");
+    return SENK_ERR_TIMEOUT;
+}
 int ctx_work(Ctx *c, size_t bytes, void **out) { return arena_get(c->work, bytes, out); }
 int ctx_events(Ctx *c) {
     if (c->dring_h) return SENK_OK;
@@ -314,6 +320,9 @@ int senk_ctx_create(int device, senk_ctx *out) {
     SENK_HIP(hipMalloc(&c.dscalars, sizeof(double) * 64));
     SENK_HIP(hipHostMalloc((void **)&c.hpinned, sizeof(double) * 64, hipHostMallocDefault));
     SENK_HIP(hipHostMalloc((void **)&c.hpinned_i, sizeof(int) * 64, hipHostMallocDefault));
+    SENK_HIP(hipHostMalloc((void **)&c.sweep_err, 64, hipHostMallocCoherent));
+    *c.sweep_err = 0;
+    SENK_HIP(hipHostGetDevicePointer((void **)&c.sweep_err_d, c.sweep_err, 0));
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) c.num_cus = prop.multiProcessorCount;
     // the no-allocation entry point's scratch array on this device (once per device); a
@@ -335,6 +344,9 @@ int senk_ctx_destroy(senk_ctx ctx) {
     if (c.dring_h) (void)hipHostFree(c.dring_h);
     (void)hipFree(c.red_partials);
     (void)hipFree(c.dscalars);
+    for (SweepVec &v : c.sweep)
+        if (v.p) (void)hipFree(v.p);
+    (void)hipHostFree(c.sweep_err);
     (void)hipHostFree(c.hpinned);
     (void)hipHostFree(c.hpinned_i);
     (void)hipStreamDestroy(c.stream);
@@ -344,7 +356,7 @@ int senk_ctx_destroy(senk_ctx ctx) {
 int senk_ctx_synchronize(senk_ctx ctx) {
     CTX_CHECK(ctx);
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
-    return SENK_OK;
+    return ctx_sweep_check(&ctx->c);
 }
 int senk_device_malloc(senk_ctx ctx, size_t bytes, void **dptr) {
     CTX_CHECK(ctx);
@@ -375,7 +387,7 @@ int senk_memcpy_dtoh(senk_ctx ctx, void *dst, const void *src, size_t bytes) {
     if (!bytes) return SENK_OK;
     SENK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->c.stream));
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
-    return SENK_OK;
+    return ctx_sweep_check(&ctx->c);
 }
 int senk_memcpy_dtod(senk_ctx ctx, void *dst, const void *src, size_t bytes) {
     CTX_CHECK(ctx);
@@ -519,7 +531,7 @@ int senk_spmv_sellcs_f32(senk_ctx ctx, const senk_sellcs *d, const float *dx, fl
         if (N % bsize) return SENK_ERR_DIVISIBILITY;                                                             \
         if (cptr[cnum] * bsize > N) return SENK_ERR_ARG;                                                         \
         Schedule s = colors(cptr, cnum, bsize);                                                                  \
-        return launch_sptrsv<T>(&ctx->c, s, UP, drptr, dcind, dval, dx, dy, nullptr, nullptr);                   \
+        return launch_sptrsv<T>(&ctx->c, s, UP, N, drptr, dcind, dval, dx, dy, nullptr, nullptr);                \
     }
 TRSV_ABMC(senk_sptrsv_csr_l_abmc_f64, double, false)
 TRSV_ABMC(senk_sptrsv_csr_u_abmc_f64, double, true)
@@ -551,12 +563,18 @@ int senk_trsv_plan_create(senk_ctx ctx, const int *rptr, const int *cind, int N,
     std::vector<int> blk;
     p->s.bsize = 1;
     p->s.nlev = host::levels(rptr, cind, N, 1, upper != 0, p->s.lev_ptr, blk);
-    const int st = upload(ctx, &p->s.dblk, blk.data(), blk.size());
+    std::vector<int> seq, pos;
+    sweep_sequence(p->s, blk, upper != 0, &p->s.streams, &p->s.seq_waves, seq, pos);
+    p->s.seq_upper = upper != 0;
+    for (int i = 0; i < N; i++) p->s.max_ext = std::max(p->s.max_ext, rptr[i + 1] - rptr[i] - (upper ? 1 : 0));
+    int st = upload(ctx, &p->s.dblk, blk.data(), blk.size());
+    if (st == SENK_OK) st = upload(ctx, &p->s.dseq, seq.data(), seq.size());
+    if (st == SENK_OK) st = upload(ctx, &p->s.dpos, pos.data(), pos.size());
+    if (st == SENK_OK && hipStreamSynchronize(ctx->c.stream) != hipSuccess) st = SENK_ERR_HIP;
     if (st != SENK_OK) {
-        delete p;
+        (void)senk_trsv_plan_destroy(p);
         return st;
     }
-    SENK_HIP(hipStreamSynchronize(ctx->c.stream));
     *out = p;
     return SENK_OK;
 }
@@ -564,6 +582,8 @@ int senk_trsv_plan_levels(senk_trsv_plan plan) { return plan ? plan->s.nlev : -1
 int senk_trsv_plan_destroy(senk_trsv_plan plan) {
     if (!plan) return SENK_ERR_ARG;
     (void)hipFree(plan->s.dblk);
+    (void)hipFree(plan->s.dseq);
+    (void)hipFree(plan->s.dpos);
     delete plan;
     return SENK_OK;
 }
@@ -573,7 +593,8 @@ static int plan_trsv(senk_ctx ctx, senk_trsv_plan plan, bool upper, const T *dva
                      const int *drptr, const T *dx, T *dy, int N) {
     CTX_CHECK(ctx);
     if (!plan || N < 0) return SENK_ERR_ARG;
-    return launch_sptrsv<T>(&ctx->c, plan->s, upper, drptr, dcind, dval, dx, dy, nullptr, nullptr);
+    return launch_sptrsv<T>(&ctx->c, plan->s, upper, plan->s.lev_ptr[plan->s.nlev], drptr, dcind, dval, dx, dy,
+                            nullptr, nullptr);
 }
 extern "C" {
 int senk_sptrsv_csr_l_f64(senk_ctx ctx, senk_trsv_plan plan, const double *dval, const int *dcind, const int *drptr,
@@ -878,6 +899,7 @@ static int finish(senk_ctx ctx, const MatView &A, const double *db, const double
     double tr = 0;
     SENK_TRY(true_relres(&ctx->c, A, db, dx, nrm_b, &tr));
     res->true_relres = tr;
+    SENK_TRY(ctx_sweep_check(&ctx->c));
     return res->status;
 }
 static int raw_mat(senk_ctx ctx, const double *dval, const int *dcind, const int *drptr, int N, MatView *A) {

@@ -47,6 +47,14 @@ __device__ __forceinline__ double wave_sum(double v) {
     return __hiloint2double(hi, lo);
 }
 
+// Orders this wave's LDS writes before its later LDS reads of other lanes' data (for
+// buffers of one wave, where no workgroup barrier is needed).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Sum over a workgroup of kBlock threads; all threads get the total.  `sh` must hold
 // kWavesPerBlock doubles and is free again on return.
 __device__ __forceinline__ double block_sum(double v, double *sh) {

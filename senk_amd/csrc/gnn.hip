@@ -169,13 +169,6 @@ __global__ __launch_bounds__(kBlock) void k_gnn_sigma(const double *P, int B, in
         sc[1] = sg > 0 ? 1.0 / sg : 0.0;
     }
 }
-// Orders this wave's LDS writes before its later LDS reads of other lanes' data (the
-// buffers below are per wave, so no workgroup barrier is needed).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 // layer 1, one thread per node (two tiles per wave); a wave's 64 node records go out
 // through the LDS so that consecutive lanes store consecutive 16 bytes
 __global__ __launch_bounds__(kBlock) void k_gnn_l1(int N, const int *__restrict__ tptr,

@@ -45,6 +45,15 @@ constexpr int kRedMaxBlocks = 1024;  // workgroups of a reducing pass
 constexpr int kRedMaxK = 40;          // simultaneous dot products per pass
 constexpr int kRedSlots = 8;          // independent partial buffers
 
+// One of the two vectors through which the single-launch solves on caller arrays publish
+// their rows (trsv_csr.hip): `clean` leading elements of `width` bytes held the sentinel
+// before its last use as the output, which wrote the first `dirty` of them (0: reset since).
+struct SweepVec {
+    void *p = nullptr;
+    size_t bytes = 0, clean = 0, dirty = 0;
+    int width = 0;
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -62,10 +71,20 @@ struct Ctx {
     // and device addresses), 8 slots of 4 ints: {sequence number, stop flag} in the first 8
     // bytes of each
     int *dring_h = nullptr, *dring_d = nullptr;
+    // single-launch solves on caller arrays: the two vectors (grown on demand, freed with the
+    // context), the one the next solve publishes in, and the time-out word in coherent
+    // pinned memory (host and device address)
+    SweepVec sweep[2];
+    int sweep_cur = 0;
+    unsigned *sweep_err = nullptr, *sweep_err_d = nullptr;
     unsigned dseq = 0;  // last sequence number handed out for the ring (runs on across solves)
 };
 // Creates the context's reusable events and pinned ring on first use.
 int ctx_events(Ctx *c);
+
+// SENK_ERR_TIMEOUT (once) if a single-launch solve on caller arrays gave up a wait; the
+// stream must be synchronised.
+int ctx_sweep_check(Ctx *c);
 
 int ctx_work(Ctx *c, size_t bytes, void **out);
 int ctx_outer(Ctx *c, size_t bytes, void **out);
@@ -80,6 +99,12 @@ struct Schedule {
     int nlev = 0;
     std::vector<int> lev_ptr;  // host
     int *dblk = nullptr;       // device, optional
+    // plans (bsize 1, dblk): the rows in the order of the single-launch solve, `streams`
+    // streams of `seq_waves` waves of 64 rows (device; -1: none) and each row's place in it,
+    // for upper = seq_upper solves
+    int *dseq = nullptr, *dpos = nullptr;
+    int streams = 0, seq_waves = 0, max_ext = 0;  // max_ext: most off-diagonal entries of a row
+    bool seq_upper = false;
 };
 
 // A triangular factor rearranged for the scheduled solve (trsv_sell.hip): per level,
@@ -183,8 +208,15 @@ int launch_spmv_sell(Ctx *c, int N, int C, int nslices, const int *wid, const in
                      long long slots = -1);  // stored slots (wid[nslices] * C) when known
 
 template <typename T>
-int launch_sptrsv(Ctx *c, const Schedule &s, bool upper, const int *rptr, const int *cind, const T *val,
+int launch_sptrsv(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr, const int *cind, const T *val,
                   const T *x, T *y, const double *in_scale, const int *stop_flag);
+// The same in one launch (trsv_csr.hip) where the schedule allows it (*done).
+template <typename T>
+int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr, const int *cind, const T *val,
+                     const T *x, T *y, const double *in_scale, const int *stop, bool *done);
+// Rows blk of a level schedule (bsize 1) in the order of the single-launch solve.
+void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, int *streams, int *waves,
+                    std::vector<int> &seq, std::vector<int> &pos);
 template <typename T>
 int launch_sptrsv_bcsr(Ctx *c, const Schedule &s, bool upper, int bnl, int bnw, const int *brptr,
                        const int *bcind, const T *bval, const T *x, T *y);

@@ -282,7 +282,10 @@ template int launch_spmv_bcsr<float>(Ctx *, int, int, int, const int *, const in
                                      float *);
 
 // =============================================================== SpTRSV (CSR)
-// One launch per schedule level.  Packed form (BS | 64): one lane per row, the BS rows
+// Schedules that the single launch of trsv_csr.hip takes go there (launch_sptrsv); what
+// follows are the launches per level for the others (block lists of several rows a block,
+// blocks that do not divide 64, more than 256 colors, colors short of N, no memory for the
+// sweep vectors).  Packed form (BS | 64): one lane per row, the BS rows
 // of a block are consecutive lanes of one wave.
 //  phase 1: each lane subtracts the entries of its row that lie outside its block
 //           (earlier levels, already final) in CSR order;
@@ -513,8 +516,11 @@ __global__ __launch_bounds__(64) void k_sptrsv_wave(int nblk, int blk0, const in
 }
 
 template <typename T>
-int launch_sptrsv(Ctx *c, const Schedule &s, bool upper, const int *rptr, const int *cind, const T *val,
+int launch_sptrsv(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr, const int *cind, const T *val,
                   const T *x, T *y, const double *in_scale, const int *stop_flag) {
+    bool done = false;
+    SENK_TRY(launch_csr_sweep<T>(c, s, upper, N, rptr, cind, val, x, y, in_scale, stop_flag, &done));
+    if (done) return SENK_OK;
     const int BS = s.bsize;
     const bool packed = BS <= 64 && (64 % BS) == 0;
     for (int step = 0; step < s.nlev; step++) {
@@ -584,9 +590,9 @@ int launch_sptrsv(Ctx *c, const Schedule &s, bool upper, const int *rptr, const 
     }
     return SENK_OK;
 }
-template int launch_sptrsv<double>(Ctx *, const Schedule &, bool, const int *, const int *, const double *,
+template int launch_sptrsv<double>(Ctx *, const Schedule &, bool, int, const int *, const int *, const double *,
                                    const double *, double *, const double *, const int *);
-template int launch_sptrsv<float>(Ctx *, const Schedule &, bool, const int *, const int *, const float *,
+template int launch_sptrsv<float>(Ctx *, const Schedule &, bool, int, const int *, const int *, const float *,
                                   const float *, float *, const double *, const int *);
 
 // =============================================================== SpTRSV (BCSR)

@@ -550,8 +550,8 @@ int prec_apply(Ctx *c, const PrecView &M, const T *in, const double *in_scale, T
         } else if (layout_has<T>(M.lt) && layout_has<T>(M.ut)) {
             SENK_TRY(launch_ilu_layout<T>(c, M.lts, *M.lt, M.uts, *M.ut, in, out, in_scale, stop));
         } else {
-            SENK_TRY(launch_sptrsv<T>(c, M.ls, false, M.lrptr, M.lcind, lv, in, out, in_scale, stop));
-            SENK_TRY(launch_sptrsv<T>(c, M.us, true, M.urptr, M.ucind, uv, out, out, nullptr, stop));
+            SENK_TRY(launch_sptrsv<T>(c, M.ls, false, N, M.lrptr, M.lcind, lv, in, out, in_scale, stop));
+            SENK_TRY(launch_sptrsv<T>(c, M.us, true, N, M.urptr, M.ucind, uv, out, out, nullptr, stop));
         }
     } else if (M.kind == 2) {
         const T *lv = std::is_same<T, double>::value ? (const T *)M.bl64 : (const T *)M.bl32;

@@ -1,0 +1,546 @@
+// Single-launch triangular solves on the caller's own CSR / BCSR factors (the colored,
+// planned and block entry points and the driver twins; factors held by a preconditioner
+// handle use the sliced layout of trsv_sell.hip).
+//
+// One launch solves a whole triangle: a row's value is published in a context-owned vector
+// z that starts all-sentinel (sweep.hpp), a gather waits until the row it reads is
+// published, and the value also goes to the caller's y with a plain store.  The launch
+// resets the context's other vector to the sentinel for the next solve, so no fill kernel
+// runs.  x may alias y: only a row's own x is read, before its y is written.
+//
+// Workgroup b belongs to stream b mod 8, the XCD the dispatcher hands it to, and holds the
+// stream's ticket b / 8; stream x solves the x-th eighth of every level (in an ABMC order a
+// band of the domain), so most gathers are served by the XCD's own L2.  Progress: every
+// stream takes its rows level by level, so the unfinished row of the lowest level waits on
+// nothing unfinished, and the first unfinished workgroup of its stream, all earlier ones of
+// that XCD's dispatcher being finished, is resident or next.  Any other order ends in the
+// bounded poll, which raises the context's time-out word, not in a hang.
+//
+// Per row the operations and their order are the sequential solve's: the same bits.
+#include "sweep.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace senk_amd {
+
+// Levels of a schedule in solve order (a kernel argument): first ticket, first unit (row or
+// block) and unit count of each.
+constexpr int kSweepMaxLevels = 256;
+struct SweepLevels {
+    int n;
+    int ticket[kSweepMaxLevels], unit0[kSweepMaxLevels], units[kSweepMaxLevels];
+};
+
+namespace {
+constexpr int kCsrWaves = 4;  // waves per workgroup, each with rows (and staged entries) of its own
+// Polls before a wait gives up (a second or more), and how often it looks whether another
+// wait has already given up.
+constexpr int kCsrSpinLimit = 1 << 20, kCsrSpinCheck = 1 << 12;
+
+// Waits until every row cc[q] (on[q]) is published in z, its bits in yb.  While a wave waits
+// it polls one row only, the first one still missing of its first waiting lane; when that one
+// is there it reads all the missing ones again.  (All of them at every poll: up to 64 x CH
+// separate lines a poll from every resident wave, which kept the memory system busy enough to
+// slow down the rows waited for.)  Polls take the XCD's own L2 and the device-coherent level
+// in turn: the first sees a row of the same XCD sooner, the second rows of the others.
+template <typename T, int CH>
+__device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], const bool (&on)[CH],
+                                           typename Bits<T>::U (&yb)[CH], unsigned *err) {
+    using U = typename Bits<T>::U;
+    int want = -1;  // the first missing row of this lane
+#pragma unroll
+    for (int q = CH - 1; q >= 0; q--)
+        if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
+    unsigned long long b = __ballot(want >= 0);
+    for (int spin = 0; b;) {
+        const T *p = z + __builtin_amdgcn_readlane(want, __ffsll((long long)b) - 1);
+        while ((spin & 1 ? load_local(p) : load_agent(p)) == Bits<T>::kSentinel) {
+            spin++;
+            if (spin >= kCsrSpinLimit ||
+                ((spin & (kCsrSpinCheck - 1)) == 0 &&
+                 __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+                __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                return;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        want = -1;
+        U nb[CH];
+#pragma unroll
+        for (int q = 0; q < CH; q++)
+            if (on[q] && yb[q] == Bits<T>::kSentinel) nb[q] = load_agent(z + cc[q]);
+#pragma unroll
+        for (int q = CH - 1; q >= 0; q--)
+            if (on[q] && yb[q] == Bits<T>::kSentinel) {
+                yb[q] = nb[q];
+                if (nb[q] == Bits<T>::kSentinel) want = cc[q];
+            }
+        b = __ballot(want >= 0);
+    }
+}
+
+// Level of ticket j (uniform): the last l with ticket[l] <= j.
+__device__ __forceinline__ int level_of(const SweepLevels &lv, int j) {
+    int lo = 0, hi = lv.n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (lv.ticket[mid] <= j) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+// The wave's slice (of `per` units) of its stream's band of level l, or -1.
+__device__ __forceinline__ int band_slice(const SweepLevels &lv, int l, int j, int xs, int per) {
+    const int ns = (lv.units[l] + per - 1) / per;
+    const int lo = (int)((long long)ns * xs / kXcds), end = (int)((long long)ns * (xs + 1) / kXcds);
+    const int sl = lo + (j - lv.ticket[l]) * kCsrWaves + (int)(threadIdx.x >> 6);
+    return sl < end ? sl : -1;
+}
+
+// ------------------------------------------------------------------ CSR, colored
+// One lane per row, the BS rows of a block in consecutive lanes (BS | 64).  The wave copies
+// its rows' slice of the factor into LDS with coalesced loads (a slice of more than
+// kCsrCap entries is read in place), then per row: the entries outside the block in rounds
+// of 8 gathers, then BS steps inside the block, each finished row broadcast in the wave.
+// Bound by the levels' dependent chain (publish, poll, in-block steps), not by bytes.
+template <typename T>
+constexpr int kCsrCap = 10 * 1024 / (int)(sizeof(T) + sizeof(int));
+
+template <typename T, int BS, bool UPPER, typename FC, typename FV>
+__device__ __forceinline__ T solve_row(T t, int s, int e, bool active, int base, const T *z, unsigned *err, FC C,
+                                       FV V) {
+    using U = typename Bits<T>::U;
+    constexpr int CH = 8;
+    const int r = (int)(threadIdx.x & 63) % BS;
+    T dinv = 0;
+    if (UPPER && active) dinv = V(s);
+    int k = UPPER ? e - 1 : s;
+    bool go = active;
+    while (__ballot(go)) {
+        int cc[CH];
+        bool on[CH];
+        T vv[CH];
+        U yb[CH];
+        int cnt = 0;
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            const int i = UPPER ? k - q : k + q;
+            const bool in = go && (UPPER ? i > s : i < e);
+            cc[q] = in ? C(i) : 0;
+            on[q] = in && (UPPER ? cc[q] >= base + BS : cc[q] < base) && (q == 0 || on[q > 0 ? q - 1 : 0]);
+            if (on[q]) {
+                vv[q] = V(i);
+                cnt++;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < CH; q++)
+            if (on[q]) yb[q] = load_local(z + cc[q]);
+        await_rows<T, CH>(z, cc, on, yb, err);
+#pragma unroll
+        for (int q = 0; q < CH; q++)
+            if (on[q]) t -= vv[q] * __builtin_bit_cast(T, yb[q]);
+        k += UPPER ? -cnt : cnt;
+        go = on[CH - 1];
+    }
+    if constexpr (BS == 1) {
+        if (UPPER) t = t * dinv;
+    } else if constexpr (BS <= 16) {
+        // mask of the in-block columns (ascending for L, descending for U); the entry of
+        // column c is then found by counting, so every value is read before the steps
+        unsigned mk = 0;
+        bool more = active;
+        int prev = UPPER ? BS : -1;
+#pragma unroll
+        for (int q = 0; q < BS; q++) {
+            const int i = UPPER ? k - q : k + q;
+            const int c = more && (UPPER ? i > s : i < e) ? C(i) - base : (UPPER ? BS : -1);
+            more = more && (UPPER ? (c < prev && c >= 0) : (c > prev && c < BS));
+            if (more) mk |= 1u << c;
+            prev = c;
+        }
+        T iv[BS];
+#pragma unroll
+        for (int c = 0; c < BS; c++) {
+            const unsigned before = UPPER ? mk >> (c + 1) : mk & ((1u << c) - 1);
+            const int p = __popc(before);
+            iv[c] = (mk >> c) & 1 ? V(UPPER ? k - p : k + p) : T(0);
+        }
+#pragma unroll
+        for (int i = 0; i < BS; i++) {
+            const int c = UPPER ? BS - 1 - i : i;
+            if (UPPER && r == c) t = t * dinv;
+            const T yc = block_bcast<BS>(t, c);
+            if ((mk >> c) & 1) t -= iv[c] * yc;
+        }
+    } else {
+        // the next in-block entry, loaded one ahead of the step that takes it
+        const int lim = UPPER ? s : e;
+        auto has = [&](int i) { return active && (UPPER ? i > lim : i < lim); };
+        int nc = has(k) ? C(k) : -1;
+        T nv = has(k) ? V(k) : T(0);
+#pragma unroll
+        for (int i = 0; i < BS; i++) {
+            const int c = UPPER ? BS - 1 - i : i;
+            if (UPPER && r == c) t = t * dinv;
+            const T yc = block_bcast<BS>(t, c);
+            if (nc == base + c) {
+                t -= nv * yc;
+                k += UPPER ? -1 : 1;
+                nc = has(k) ? C(k) : -1;
+                nv = has(k) ? V(k) : T(0);
+            }
+        }
+    }
+    return t;
+}
+
+template <typename T, int BS, bool UPPER>
+__global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, const int *__restrict__ rptr,
+                                                              const int *__restrict__ cind,
+                                                              const T *__restrict__ val, const T *x, T *y, T *z,
+                                                              T *reset, const double *__restrict__ in_scale,
+                                                              unsigned *err, const int *__restrict__ stop) {
+    __shared__ T sv[kCsrWaves][kCsrCap<T>];
+    __shared__ int sc[kCsrWaves][kCsrCap<T>];
+    const int xs = (int)(blockIdx.x % kXcds), j = (int)(blockIdx.x / kXcds);
+    const int l = level_of(lv, j), sl = __builtin_amdgcn_readfirstlane(band_slice(lv, l, j, xs, 64));
+    if (sl < 0) return;
+    const int wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    const int r0 = lv.unit0[l] + sl * 64, nr = min(64, lv.units[l] - sl * 64);
+    const int row = r0 + lane;
+    const bool active = lane < nr;
+    const int stopped = stop ? *stop : 0;
+    int s = 0, e = 0;
+    T t = 0;
+    if (active) {
+        s = rptr[row];
+        e = rptr[row + 1];
+        t = x[row];
+        reset[row] = __builtin_bit_cast(T, Bits<T>::kSentinel);
+    }
+    if (stopped) return;
+    if (!UPPER && in_scale && active) t = (T)((double)t * *in_scale);
+    const int e0 = __builtin_amdgcn_readlane(s, 0), e1 = __builtin_amdgcn_readlane(e, nr - 1);
+    const int base = row - lane % BS;
+    if (e1 - e0 <= kCsrCap<T>) {
+        const int n = e1 - e0;
+        for (int q0 = lane; q0 < n; q0 += 64 * 4) {
+            T v[4];
+            int c[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (q0 + 64 * u < n) {
+                    v[u] = val[e0 + q0 + 64 * u];
+                    c[u] = cind[e0 + q0 + 64 * u];
+                }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (q0 + 64 * u < n) {
+                    sv[wv][q0 + 64 * u] = v[u];
+                    sc[wv][q0 + 64 * u] = c[u];
+                }
+        }
+        wave_lds_sync();
+        t = solve_row<T, BS, UPPER>(t, s - e0, e - e0, active, base, z, err, [&](int i) { return sc[wv][i]; },
+                                    [&](int i) { return sv[wv][i]; });
+    } else {
+        t = solve_row<T, BS, UPPER>(t, s, e, active, base, z, err, [&](int i) { return cind[i]; },
+                                    [&](int i) { return val[i]; });
+    }
+    if (active) {
+        store_agent(z + row, canonical(t));
+        y[row] = t;
+    }
+}
+
+// ------------------------------------------------------------------ CSR, planned (level lists)
+// Rows of a level schedule (bsize 1): seq holds the rows in stream order, wave w of stream x
+// taking seq[(w * streams + x) * 64 + lane] (-1: none).  Rows of several levels may share a
+// wave, so no lane waits for another: every lane polls for its own entries, and a lane whose
+// round is complete subtracts it and goes on or publishes its row, whatever the others wait
+// for.  Rows are published by their place in seq (pos), not by row: the rows that a level's
+// consecutive rows wait for are then close together, and a poll touches a few lines instead
+// of one per entry (published by row, every resident wave's polls kept the memory system
+// busy: 61x64x67 7-point grid, 190 levels, L + U in FP64 1352 us, 581 by place; one launch
+// per level 1746).  What is left is one publish-and-poll round trip per level, about 1.5 us.
+template <typename T, bool UPPER, int CH>
+__global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restrict__ seq,
+                                                 const int *__restrict__ pos,
+                                                 const int *__restrict__ rptr, const int *__restrict__ cind,
+                                                 const T *__restrict__ val, const T *x, T *y, T *z, T *reset,
+                                                 const double *__restrict__ in_scale, unsigned *err,
+                                                 const int *__restrict__ stop) {
+    using U = typename Bits<T>::U;
+    const int xs = (int)(blockIdx.x % kXcds), w = (int)(blockIdx.x / kXcds);
+    if (xs >= streams) return;
+    const int mine = (w * streams + xs) * 64 + (int)(threadIdx.x & 63);
+    const int row = seq[mine];
+    const int stopped = stop ? *stop : 0;
+    bool act = row >= 0;
+    int s = 0, e = 0, k = 0;
+    T t = 0, dinv = 0;
+    if (act) {
+        s = rptr[row];
+        e = rptr[row + 1];
+        t = x[row];
+    }
+    reset[mine] = __builtin_bit_cast(T, Bits<T>::kSentinel);
+    if (stopped) return;
+    if (act) {
+        if (UPPER) dinv = val[s];
+        else if (in_scale) t = (T)((double)t * *in_scale);
+        k = UPPER ? e - 1 : s;
+    }
+    int cc[CH];
+    bool on[CH];
+    T vv[CH];
+    U yb[CH];
+    auto round = [&]() {
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            const int i = UPPER ? k - q : k + q;
+            const bool in = act && (UPPER ? i > s : i < e);
+            cc[q] = in ? cind[i] : 0;
+            vv[q] = in ? val[i] : T(0);
+            on[q] = in && (UPPER ? cc[q] > row : cc[q] < row) && (q == 0 || on[q > 0 ? q - 1 : 0]);
+        }
+#pragma unroll
+        for (int q = 0; q < CH; q++) cc[q] = on[q] ? pos[cc[q]] : 0;
+#pragma unroll
+        for (int q = 0; q < CH; q++) yb[q] = on[q] ? load_local(z + cc[q]) : U(0);
+    };
+    round();
+    for (int spin = 0; __ballot(act); spin++) {
+        bool pend = false;
+#pragma unroll
+        for (int q = 0; q < CH; q++) pend |= on[q] && yb[q] == Bits<T>::kSentinel;
+        if (__ballot(act && !pend)) {
+            spin = 0;
+            if (act && !pend) {
+                int cnt = 0;
+#pragma unroll
+                for (int q = 0; q < CH; q++)
+                    if (on[q]) {
+                        t -= vv[q] * __builtin_bit_cast(T, yb[q]);
+                        cnt++;
+                    }
+                k += UPPER ? -cnt : cnt;
+                if (on[CH - 1]) {
+                    round();
+                } else {
+                    if (UPPER) t = t * dinv;
+                    store_agent(z + mine, canonical(t));
+                    y[row] = t;
+                    act = false;
+                }
+            }
+            continue;
+        }
+        if (spin >= kCsrSpinLimit ||
+            ((spin & (kCsrSpinCheck - 1)) == kCsrSpinCheck - 1 &&
+             __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+            // give up: publish a NaN so that the rows behind this one end too
+            if (act) {
+                __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                t = __builtin_nan("");
+                store_agent(z + mine, canonical(t));
+                y[row] = t;
+            }
+            return;
+        }
+        __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+        for (int q = 0; q < CH; q++)
+            if (act && on[q] && yb[q] == Bits<T>::kSentinel)
+                yb[q] = (spin & 1) ? load_agent(z + cc[q]) : load_local(z + cc[q]);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_fill_sentinel2(size_t n, T *p) {
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
+        p[i] = __builtin_bit_cast(T, Bits<T>::kSentinel);
+}
+}  // namespace
+
+// ------------------------------------------------------------------ host side
+// The sweep vectors of the next solve of n rows: *z all-sentinel (filled here where the
+// last solves left less than that), *reset the vector the launch must fill in its first n
+// rows.  false: no memory (the caller takes its launch-per-level path).
+template <typename T>
+static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
+    SweepVec *v = c->sweep;
+    *ok = false;
+    const size_t bytes = n * sizeof(T);
+    if (!c->sweep_err) return SENK_OK;
+    if (v[0].bytes < bytes) {
+        // grown while nothing of this context runs on it; allowed during a stream capture
+        // of the calling thread (the context's stream is never captured)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        SENK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        int st = hipStreamSynchronize(c->stream) == hipSuccess ? SENK_OK : SENK_ERR_HIP;
+        bool got = st == SENK_OK;
+        for (int i = 0; i < 2 && got; i++) {
+            if (v[i].p) (void)hipFree(v[i].p);
+            v[i] = SweepVec{};
+            got = hipMalloc(&v[i].p, bytes) == hipSuccess;
+            if (!got) v[i].p = nullptr;
+        }
+        if (!got) {
+            (void)hipGetLastError();
+            for (int i = 0; i < 2; i++) {
+                if (v[i].p) (void)hipFree(v[i].p);
+                v[i] = SweepVec{};
+            }
+        } else {
+            v[0].bytes = v[1].bytes = bytes;
+        }
+        SENK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        if (st) return st;
+        if (!got) return SENK_OK;
+    }
+    SweepVec &u = v[c->sweep_cur], &o = v[c->sweep_cur ^ 1];
+    if (u.width != (int)sizeof(T) || u.clean < n) {
+        k_fill_sentinel2<T><<<(int)std::min<size_t>((n + kBlock - 1) / kBlock, 2048), kBlock, 0, c->stream>>>(
+            n, (T *)u.p);
+        SENK_LAUNCH_CHECK();
+        u.width = (int)sizeof(T);
+        u.clean = n;
+    }
+    // what this launch leaves: u written in its first n rows, o clean in them (and beyond,
+    // where o's last solve was no longer)
+    u.dirty = n;
+    if (o.width == (int)sizeof(T) && n >= o.dirty) o.clean = std::max(o.clean, n);
+    else o.clean = n;
+    o.width = (int)sizeof(T);
+    o.dirty = 0;
+    *z = (T *)u.p;
+    *reset = (T *)o.p;
+    c->sweep_cur ^= 1;
+    *ok = true;
+    return SENK_OK;
+}
+
+// Average rows per level below which a plan's rows go through one stream, i.e. one XCD: a
+// thin level has no use for the others' bandwidth, and its waits stay on one die.  L + U in
+// FP64, one / eight streams: 7-point 12^3 (50 rows a level) 75 / 102 us, 24^3 (197) 165 /
+// 203, 40^3 (542) 315 / 350, 61x64x67 (1377) 637 / 581; 27-point 38^3 (209) 1341 / 1437.
+constexpr double kPlanOneStream = 800;
+void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, int *streams, int *waves,
+                    std::vector<int> &seq, std::vector<int> &pos) {
+    const int S = s.nlev > 0 && (double)blk.size() / s.nlev < kPlanOneStream ? 1 : kXcds;
+    std::vector<int> of[kXcds];
+    for (int step = 0; step < s.nlev; step++) {
+        const int l = upper ? s.nlev - 1 - step : step;
+        const long long a = s.lev_ptr[l], n = s.lev_ptr[l + 1] - a;
+        for (int x = 0; x < S; x++)
+            of[x].insert(of[x].end(), blk.begin() + (a + n * x / S), blk.begin() + (a + n * (x + 1) / S));
+    }
+    size_t w = 0;
+    for (int x = 0; x < S; x++) w = std::max(w, (of[x].size() + 63) / 64);
+    seq.assign(w * S * 64, -1);
+    pos.assign(blk.size(), 0);
+    for (int x = 0; x < S; x++)
+        for (size_t i = 0; i < of[x].size(); i++) {
+            const size_t p = ((i / 64) * S + x) * 64 + i % 64;
+            seq[p] = of[x][i];
+            pos[of[x][i]] = (int)p;
+        }
+    *streams = S;
+    *waves = (int)w;
+}
+
+// The level table of a schedule in solve order; units of a level: rows or blocks, `per` of
+// them in a wave's slice.
+static bool sweep_levels(const Schedule &s, bool upper, int scale, int per, SweepLevels *lv, int *tickets) {
+    lv->n = 0;
+    int tk = 0;
+    for (int step = 0; step < s.nlev; step++) {
+        const int l = upper ? s.nlev - 1 - step : step;
+        const int nb = s.lev_ptr[l + 1] - s.lev_ptr[l];
+        if (nb < 0) return false;
+        if (nb == 0) continue;
+        if (lv->n >= kSweepMaxLevels) return false;
+        lv->ticket[lv->n] = tk;
+        lv->unit0[lv->n] = s.lev_ptr[l] * scale;
+        lv->units[lv->n] = nb * scale;
+        lv->n++;
+        const int ns = (nb * scale + per - 1) / per;
+        int most = 0;
+        for (int x = 0; x < kXcds; x++)
+            most = std::max(most, (int)((long long)ns * (x + 1) / kXcds - (long long)ns * x / kXcds));
+        tk += (most + kCsrWaves - 1) / kCsrWaves;
+    }
+    *tickets = tk;
+    return lv->n > 0;
+}
+
+template <typename T>
+int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr, const int *cind, const T *val,
+                     const T *x, T *y, const double *in_scale, const int *stop, bool *done) {
+    *done = false;
+    const int BS = s.bsize;
+    if (BS < 1 || BS > 64 || 64 % BS || s.lev_ptr.empty() || s.lev_ptr[0] != 0 ||
+        (long long)s.lev_ptr[s.nlev] * BS != N)
+        return SENK_OK;
+    T *z = nullptr, *reset = nullptr;
+    if (s.dblk) {
+        if (BS != 1 || !s.dseq || !s.dpos || s.seq_upper != upper) return SENK_OK;
+        bool ok = false;
+        SENK_TRY(sweep_vectors<T>(c, (size_t)s.seq_waves * s.streams * 64, &z, &reset, &ok));
+        if (!ok) return SENK_OK;
+        const int grid = kXcds * s.seq_waves;
+        // rounds of 4 where no row has more entries, else of 16: a second round costs its own
+        // chain of dependent loads after the last row of the first is there
+#define SENK_CSR_ROWS(UP, CH)                                                                                      \
+    k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.streams, s.dseq, s.dpos, rptr, cind, val, x, y, z, reset, \
+                                                      UP ? nullptr : in_scale, c->sweep_err_d, stop)
+        if (upper && s.max_ext <= 4) SENK_CSR_ROWS(true, 4);
+        else if (upper) SENK_CSR_ROWS(true, 16);
+        else if (s.max_ext <= 4) SENK_CSR_ROWS(false, 4);
+        else SENK_CSR_ROWS(false, 16);
+#undef SENK_CSR_ROWS
+        SENK_LAUNCH_CHECK();
+        *done = true;
+        return SENK_OK;
+    }
+    SweepLevels lv;
+    int tickets = 0;
+    if (!sweep_levels(s, upper, BS, 64, &lv, &tickets)) return SENK_OK;
+    bool ok = false;
+    SENK_TRY(sweep_vectors<T>(c, (size_t)N, &z, &reset, &ok));
+    if (!ok) return SENK_OK;
+    const int grid = kXcds * tickets;
+#define SENK_CSR_SWEEP(B)                                                                                        \
+    case B:                                                                                                      \
+        if (upper)                                                                                               \
+            k_csr_sweep<T, B, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z, reset, \
+                                                                            nullptr, c->sweep_err_d, stop);      \
+        else                                                                                                     \
+            k_csr_sweep<T, B, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z,       \
+                                                                             reset, in_scale, c->sweep_err_d,    \
+                                                                             stop);                              \
+        break;
+    switch (BS) {
+        SENK_CSR_SWEEP(1)
+        SENK_CSR_SWEEP(2)
+        SENK_CSR_SWEEP(4)
+        SENK_CSR_SWEEP(8)
+        SENK_CSR_SWEEP(16)
+        SENK_CSR_SWEEP(32)
+        SENK_CSR_SWEEP(64)
+        default: return SENK_ERR_UNSUPPORTED;
+    }
+#undef SENK_CSR_SWEEP
+    SENK_LAUNCH_CHECK();
+    *done = true;
+    return SENK_OK;
+}
+template int launch_csr_sweep<double>(Ctx *, const Schedule &, bool, int, const int *, const int *, const double *,
+                                      const double *, double *, const double *, const int *, bool *);
+template int launch_csr_sweep<float>(Ctx *, const Schedule &, bool, int, const int *, const int *, const float *,
+                                     const float *, float *, const double *, const int *, bool *);
+
+}  // namespace senk_amd

@@ -1,0 +1,145 @@
+"""Single-launch triangular solves on the caller's CSR factors (ABMC colors and plans).
+
+Every row keeps the sequential solve's operations and their order, so the results must be the
+oracle's sequential solve bit for bit, whatever solves of other sizes and types ran before
+on the context (the solves share two vectors that each leaves ready for the next).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import senk_amd as S
+from oracle import oracle as O
+from tests.helpers import abmc_system, ilu_factors
+
+pytestmark = pytest.mark.gpu
+
+
+def _seq(L, U, x):
+    """The oracle's sequential solves L, then U, in x's type."""
+    N, s = len(x), "d" if x.dtype == np.float64 else "f"
+    yl, yu = np.zeros_like(x), np.zeros_like(x)
+    getattr(O.orc(), "or_sptrsv_l_" + s)(O.P(L[0]), O.P(L[1]), O.P(L[2]), O.P(x), O.P(yl), N)
+    getattr(O.orc(), "or_sptrsv_u_" + s)(O.P(U[0]), O.P(U[1]), O.P(U[2]), O.P(yl), O.P(yu), N)
+    return yl, yu
+
+
+def _typed(f, dt):
+    return (np.ascontiguousarray(f[0].astype(dt)), f[1], f[2])
+
+
+def _abmc_case(ctx, mat, bsize, method, dt):
+    val, cind, rptr, N = S.padding(mat[2], mat[1], mat[0], bsize, len(mat[0]) - 1)
+    sy = abmc_system(rptr, cind, val, bsize, method)
+    L, U = (_typed(f, dt) for f in ilu_factors(sy))
+    x = np.random.default_rng(N + bsize).uniform(-1, 1, N).astype(dt)
+    x[N // 3] = 0.0
+    yl, yu = _seq(L, U, x)
+    d = [ctx.array(t) for t in (*L, *U, x)]
+    s = "f64" if dt == np.float64 else "f32"
+    cp = O.P(sy["cptr"])
+    dy = ctx.zeros(N, dt)
+    S.call("senk_sptrsv_csr_l_abmc_" + s, ctx.h, *(t.p for t in d[:3]), d[6].p, dy.p, N, cp, sy["nc"], bsize)
+    t = dy.download()
+    S.call("senk_sptrsv_csr_u_abmc_" + s, ctx.h, *(t.p for t in d[3:6]), dy.p, dy.p, N, cp, sy["nc"], bsize)  # in place
+    assert np.array_equal(t, yl) and np.array_equal(dy.download(), yu)
+
+
+def _plan_case(ctx, mat, dt):
+    rptr, cind, val = mat
+    N = len(rptr) - 1
+    L, U = (_typed(f, dt) for f in ilu_factors(dict(val=val, cind=cind, rptr=rptr)))
+    x = np.random.default_rng(N).uniform(-1, 1, N).astype(dt)
+    yl, yu = _seq(L, U, x)
+    d = [ctx.array(t) for t in (*L, *U, x)]
+    s = "f64" if dt == np.float64 else "f32"
+    plans = []
+    for f, up in ((L, 0), (U, 1)):
+        p = C.c_void_p()
+        S.call("senk_trsv_plan_create", ctx.h, O.P(f[2]), O.P(f[1]), N, up, C.byref(p))
+        plans.append(p)
+    dy = d[6]  # L in place as well
+    S.call("senk_sptrsv_csr_l_" + s, ctx.h, plans[0], *(t.p for t in d[:3]), dy.p, dy.p, N)
+    t = dy.download()
+    S.call("senk_sptrsv_csr_u_" + s, ctx.h, plans[1], *(t.p for t in d[3:6]), dy.p, dy.p, N)
+    u = dy.download()
+    for p in plans:
+        S.lib().senk_trsv_plan_destroy(p)
+    assert np.array_equal(t, yl) and np.array_equal(u, yu)
+
+
+def _tridiagonal(n):
+    r = np.arange(n)
+    rows = np.concatenate([r, r[1:], r[:-1]])
+    cols = np.concatenate([r, r[1:] - 1, r[:-1] + 1])
+    vals = np.concatenate([np.full(n, 4.0), np.full(n - 1, -1.0), np.full(n - 1, -1.5)])
+    o = np.lexsort((cols, rows))
+    rptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))])
+    return rptr.astype(np.int32), cols[o].astype(np.int32), vals[o]
+
+
+# sizes around the slice of 64 rows and the ticket of 4 slices, rows of more than one round of
+# gathers, slices of more entries than the wave stages in LDS (27-point in FP64)
+@pytest.mark.parametrize("bsize", [1, 2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_abmc_in_turn_with_other_sizes(ctx, bsize, dt):
+    other = np.float32 if dt == np.float64 else np.float64
+    _abmc_case(ctx, S.gen_convdiff27(11, 10.0), bsize, "connect", dt)
+    _abmc_case(ctx, S.gen_poisson7(3, 5, 4), bsize, "simple", other)
+    _abmc_case(ctx, S.gen_vardiff7(13, 3, 4.0, 1.5), bsize, "simple", dt)
+    _abmc_case(ctx, S.gen_unstructured(2500, 5), bsize, "connect", dt)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_plans_in_turn_with_other_sizes(ctx, dt):
+    other = np.float32 if dt == np.float64 else np.float64
+    _plan_case(ctx, S.gen_poisson7(13, 9, 11), dt)        # one stream
+    _plan_case(ctx, _tridiagonal(1), other)
+    _plan_case(ctx, _tridiagonal(333), dt)                # every row waits on one of its own wave
+    _plan_case(ctx, S.gen_convdiff27(12, 10.0), dt)       # rows of 13
+    _plan_case(ctx, S.gen_unstructured(20000, 7), dt)     # long rows, several rounds
+    _plan_case(ctx, S.gen_poisson7(48, 46, 47), other)    # eight streams
+
+
+def test_non_finite_values_pass_through(ctx):
+    """An x that holds NaN (with any payload, the sentinel's too) and infinities: the solve
+    ends, and what it leaves non-finite is what the sequential solve leaves."""
+    rptr, cind, val = S.gen_poisson7(12)
+    N = len(rptr) - 1
+    sy = abmc_system(rptr, cind, val, 8)
+    L, U = ilu_factors(sy)
+    x = np.random.default_rng(4).uniform(-1, 1, N)
+    x[5], x[700] = np.inf, np.nan
+    x.view(np.uint64)[901] = 0x7FF4A5A5A5A5A5A5
+    yl, yu = _seq(L, U, x)
+    d = [ctx.array(t) for t in (*L, *U, x)]
+    dy = ctx.zeros(N)
+    cp = O.P(sy["cptr"])
+    S.call("senk_sptrsv_csr_l_abmc_f64", ctx.h, *(t.p for t in d[:3]), d[6].p, dy.p, N, cp, sy["nc"], 8)
+    assert np.array_equal(dy.download(), yl, equal_nan=True)
+    S.call("senk_sptrsv_csr_u_abmc_f64", ctx.h, *(t.p for t in d[3:6]), dy.p, dy.p, N, cp, sy["nc"], 8)
+    assert np.array_equal(dy.download(), yu, equal_nan=True)
+    _abmc_case(ctx, (rptr, cind, val), 8, "connect", np.float64)  # nothing is left behind
+
+
+def test_schedules_outside_the_single_launch(ctx):
+    """More levels than the launch's table holds, and colors that stop short of N, keep the
+    launch per level."""
+    rptr, cind, val = _tridiagonal(400)
+    N = len(rptr) - 1
+    L, U = ilu_factors(dict(val=val, cind=cind, rptr=rptr))
+    x = np.random.default_rng(2).uniform(-1, 1, N)
+    yl, yu = _seq(L, U, x)
+    d = [ctx.array(t) for t in (*L, *U, x)]
+    dy = ctx.zeros(N)
+    cptr = np.arange(N + 1, dtype=np.int32)  # one row a color
+    S.call("senk_sptrsv_csr_l_amc_f64", ctx.h, *(t.p for t in d[:3]), d[6].p, dy.p, N, O.P(cptr), N)
+    S.call("senk_sptrsv_csr_u_amc_f64", ctx.h, *(t.p for t in d[3:6]), dy.p, dy.p, N, O.P(cptr), N)
+    assert np.array_equal(dy.download(), yu)
+    # the first 200 rows only: the rest of y stays
+    dy2 = ctx.array(np.full(N, 7.0))
+    part = np.arange(201, dtype=np.int32)
+    S.call("senk_sptrsv_csr_l_amc_f64", ctx.h, *(t.p for t in d[:3]), d[6].p, dy2.p, N, O.P(part), 200)
+    out = dy2.download()
+    assert np.array_equal(out[:200], yl[:200]) and np.all(out[200:] == 7.0)
