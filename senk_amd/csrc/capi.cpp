@@ -563,13 +563,14 @@ int senk_trsv_plan_create(senk_ctx ctx, const int *rptr, const int *cind, int N,
     std::vector<int> blk;
     p->s.bsize = 1;
     p->s.nlev = host::levels(rptr, cind, N, 1, upper != 0, p->s.lev_ptr, blk);
-    std::vector<int> seq, pos;
-    sweep_sequence(p->s, blk, upper != 0, &p->s.streams, &p->s.seq_waves, seq, pos);
-    p->s.seq_upper = upper != 0;
     for (int i = 0; i < N; i++) p->s.max_ext = std::max(p->s.max_ext, rptr[i + 1] - rptr[i] - (upper ? 1 : 0));
-    int st = upload(ctx, &p->s.dblk, blk.data(), blk.size());
-    if (st == SENK_OK) st = upload(ctx, &p->s.dseq, seq.data(), seq.size());
-    if (st == SENK_OK) st = upload(ctx, &p->s.dpos, pos.data(), pos.size());
+    // one device array: the level lists, then the single-launch sequence and the rows' places
+    std::vector<int> lists;
+    sweep_sequence(p->s, blk, upper != 0, &p->s.streams, &p->s.seq_waves, lists);
+    p->s.seq_upper = upper != 0;
+    int st = upload(ctx, &p->s.dblk, lists.data(), lists.size());
+    p->s.dseq = p->s.dblk + blk.size();
+    p->s.dpos = p->s.dseq + (size_t)p->s.streams * p->s.seq_waves * 64;
     if (st == SENK_OK && hipStreamSynchronize(ctx->c.stream) != hipSuccess) st = SENK_ERR_HIP;
     if (st != SENK_OK) {
         (void)senk_trsv_plan_destroy(p);
@@ -582,8 +583,6 @@ int senk_trsv_plan_levels(senk_trsv_plan plan) { return plan ? plan->s.nlev : -1
 int senk_trsv_plan_destroy(senk_trsv_plan plan) {
     if (!plan) return SENK_ERR_ARG;
     (void)hipFree(plan->s.dblk);
-    (void)hipFree(plan->s.dseq);
-    (void)hipFree(plan->s.dpos);
     delete plan;
     return SENK_OK;
 }
@@ -641,7 +640,7 @@ static int bcsr_abmc(senk_ctx ctx, const T *dbval, const int *dbcind, const int 
     if (!cptr || cnum < 0 || bsize <= 0 || bnl <= 0 || bnw <= 0) return SENK_ERR_ARG;
     if (N % bsize || bsize % bnl || bnl % bnw) return SENK_ERR_DIVISIBILITY;
     Schedule s = colors(cptr, cnum, bsize);
-    return launch_sptrsv_bcsr<T>(&ctx->c, s, upper, bnl, bnw, dbrptr, dbcind, dbval, dx, dy);
+    return launch_sptrsv_bcsr<T>(&ctx->c, s, upper, N, bnl, bnw, dbrptr, dbcind, dbval, dx, dy);
 }
 // Sequential BCSR forms: the group-level dependency levels are computed from a host
 // copy of the block pattern on every call (the reference runs these serially too).
@@ -669,7 +668,7 @@ static int bcsr_seq(senk_ctx ctx, const T *dbval, const int *dbcind, const int *
     if (N % bnl || bnl % bnw) return SENK_ERR_DIVISIBILITY;
     Schedule s;
     SENK_TRY(bcsr_seq_schedule(ctx, dbcind, dbrptr, N, bnl, bnw, upper, &s));
-    const int st = launch_sptrsv_bcsr<T>(&ctx->c, s, upper, bnl, bnw, dbrptr, dbcind, dbval, dx, dy);
+    const int st = launch_sptrsv_bcsr<T>(&ctx->c, s, upper, N, bnl, bnw, dbrptr, dbcind, dbval, dx, dy);
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
     (void)hipFree(s.dblk);
     return st;

@@ -214,12 +214,16 @@ int launch_sptrsv(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr,
 template <typename T>
 int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr, const int *cind, const T *val,
                      const T *x, T *y, const double *in_scale, const int *stop, bool *done);
-// Rows blk of a level schedule (bsize 1) in the order of the single-launch solve.
+// Rows blk of a level schedule (bsize 1) in the order of the single-launch solve: out = blk,
+// the sequence of streams * waves * 64 rows, and each row's place in it.
 void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, int *streams, int *waves,
-                    std::vector<int> &seq, std::vector<int> &pos);
+                    std::vector<int> &out);
 template <typename T>
-int launch_sptrsv_bcsr(Ctx *c, const Schedule &s, bool upper, int bnl, int bnw, const int *brptr,
+int launch_sptrsv_bcsr(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,
                        const int *bcind, const T *bval, const T *x, T *y);
+template <typename T>
+int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,
+                      const int *bcind, const T *bval, const T *x, T *y, bool *done);
 template <typename T>
 int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *cind, const int *dpos, T *val,
                 int *derr);

@@ -596,6 +596,7 @@ template int launch_sptrsv<float>(Ctx *, const Schedule &, bool, int, const int 
                                   const float *, float *, const double *, const int *);
 
 // =============================================================== SpTRSV (BCSR)
+// The launch per level, for the schedules that the single launch of trsv_csr.hip does not take.
 // One lane per schedule block of bsize rows, walking its bnl-row groups in order with
 // the reference's column-oriented updates (senk_sparse.hpp:399-415, 436-464); the
 // group's values stay in registers.
@@ -664,9 +665,12 @@ __global__ __launch_bounds__(kBlock) void k_sptrsv_bcsr(int nblk, int blk0, cons
     }
 }
 template <typename T>
-int launch_sptrsv_bcsr(Ctx *c, const Schedule &s, bool upper, int bnl, int bnw, const int *brptr, const int *bcind,
-                       const T *bval, const T *x, T *y) {
+int launch_sptrsv_bcsr(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,
+                       const int *bcind, const T *bval, const T *x, T *y) {
     if (s.bsize % bnl) return SENK_ERR_DIVISIBILITY;
+    bool done = false;
+    SENK_TRY(launch_bcsr_sweep<T>(c, s, upper, N, bnl, bnw, brptr, bcind, bval, x, y, &done));
+    if (done) return SENK_OK;
     for (int step = 0; step < s.nlev; step++) {
         const int l = upper ? s.nlev - 1 - step : step;
         const int b0 = s.lev_ptr[l], nb = s.lev_ptr[l + 1] - b0;
@@ -684,9 +688,9 @@ int launch_sptrsv_bcsr(Ctx *c, const Schedule &s, bool upper, int bnl, int bnw, 
     }
     return SENK_OK;
 }
-template int launch_sptrsv_bcsr<double>(Ctx *, const Schedule &, bool, int, int, const int *, const int *,
+template int launch_sptrsv_bcsr<double>(Ctx *, const Schedule &, bool, int, int, int, const int *, const int *,
                                         const double *, const double *, double *);
-template int launch_sptrsv_bcsr<float>(Ctx *, const Schedule &, bool, int, int, const int *, const int *,
+template int launch_sptrsv_bcsr<float>(Ctx *, const Schedule &, bool, int, int, int, const int *, const int *,
                                        const float *, const float *, float *);
 
 // =============================================================== ILU(0) numeric

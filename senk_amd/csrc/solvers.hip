@@ -564,8 +564,8 @@ int prec_apply(Ctx *c, const PrecView &M, const T *in, const double *in_scale, T
             SENK_LAUNCH_CHECK();
             src = tmp;
         }
-        SENK_TRY(launch_sptrsv_bcsr<T>(c, M.ls, false, M.bnl, M.bnw, M.blrptr, M.blcind, lv, src, out));
-        SENK_TRY(launch_sptrsv_bcsr<T>(c, M.us, true, M.bnl, M.bnw, M.burptr, M.bucind, uv, out, out));
+        SENK_TRY(launch_sptrsv_bcsr<T>(c, M.ls, false, N, M.bnl, M.bnw, M.blrptr, M.blcind, lv, src, out));
+        SENK_TRY(launch_sptrsv_bcsr<T>(c, M.us, true, N, M.bnl, M.bnw, M.burptr, M.bucind, uv, out, out));
     } else {
         return SENK_ERR_ARG;
     }

@@ -4,6 +4,8 @@
 
 #include "dev_common.hpp"
 
+#include <type_traits>
+
 namespace senk_amd {
 
 // number of set bits of b in the lanes below this one
@@ -117,6 +119,19 @@ __device__ __forceinline__ void store_agent(T *p, T v) {
 }
 __device__ __forceinline__ float canonical(float v) { return __builtin_canonicalizef(v); }
 __device__ __forceinline__ double canonical(double v) { return __builtin_canonicalize(v); }
+// p + i; with O32 addressed as p's (uniform) base plus a 32-bit byte offset, one address
+// register per access instead of a 64-bit pair (the launch checks that every array of the
+// layout and every vector fits: i * sizeof(P) < 2^32)
+template <bool O32, typename P>
+__device__ __forceinline__ P *ixp(P *p, size_t i) {
+    if constexpr (O32) {
+        using Ch = typename std::conditional<std::is_const<P>::value, const char, char>::type;
+        return reinterpret_cast<P *>(reinterpret_cast<Ch *>(p) + (size_t)((unsigned)i * (unsigned)sizeof(P)));
+    } else {
+        return p + i;
+    }
+}
+
 // polls of one pending gather before the wave gives up and raises the time-out flag;
 // a poll takes about a microsecond, so this bounds a wait at a few seconds
 constexpr int kSweepSpinLimit = 1 << 22;

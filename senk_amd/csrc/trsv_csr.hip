@@ -39,18 +39,18 @@ constexpr int kCsrWaves = 4;  // waves per workgroup, each with rows (and staged
 constexpr int kCsrSpinLimit = 1 << 20, kCsrSpinCheck = 1 << 12;
 
 // Waits until every row cc[q] (on[q]) is published in z, its bits in yb.  While a wave waits
-// it polls one row only, the first one still missing of its first waiting lane; when that one
-// is there it reads all the missing ones again.  (All of them at every poll: up to 64 x CH
-// separate lines a poll from every resident wave, which kept the memory system busy enough to
-// slow down the rows waited for.)  Polls take the XCD's own L2 and the device-coherent level
-// in turn: the first sees a row of the same XCD sooner, the second rows of the others.
+// it polls one row only, the last one still missing of its first waiting lane (the latest
+// color); when that one is there it reads all the missing ones again.  (Polling all of them,
+// up to 64 x CH lines a poll from every resident wave, slows down the rows waited for:
+// GMRES(30) of a 64^3 system 39.7 against 36.6 ms.)  Polls take the XCD's own L2 and the
+// device-coherent level in turn: the first may see a row of the same XCD sooner, the second
+// sees those of the others.
 template <typename T, int CH>
 __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], const bool (&on)[CH],
                                            typename Bits<T>::U (&yb)[CH], unsigned *err) {
-    using U = typename Bits<T>::U;
-    int want = -1;  // the first missing row of this lane
+    int want = -1;  // the last missing row of this lane
 #pragma unroll
-    for (int q = CH - 1; q >= 0; q--)
+    for (int q = 0; q < CH; q++)
         if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
     unsigned long long b = __ballot(want >= 0);
     for (int spin = 0; b;) {
@@ -65,17 +65,13 @@ __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], cons
             }
             __builtin_amdgcn_s_sleep(1);
         }
-        want = -1;
-        U nb[CH];
 #pragma unroll
         for (int q = 0; q < CH; q++)
-            if (on[q] && yb[q] == Bits<T>::kSentinel) nb[q] = load_agent(z + cc[q]);
+            if (on[q] && yb[q] == Bits<T>::kSentinel) yb[q] = load_agent(ixp<true>(z, cc[q]));
+        want = -1;
 #pragma unroll
-        for (int q = CH - 1; q >= 0; q--)
-            if (on[q] && yb[q] == Bits<T>::kSentinel) {
-                yb[q] = nb[q];
-                if (nb[q] == Bits<T>::kSentinel) want = cc[q];
-            }
+        for (int q = 0; q < CH; q++)
+            if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
         b = __ballot(want >= 0);
     }
 }
@@ -136,7 +132,7 @@ __device__ __forceinline__ T solve_row(T t, int s, int e, bool active, int base,
         }
 #pragma unroll
         for (int q = 0; q < CH; q++)
-            if (on[q]) yb[q] = load_local(z + cc[q]);
+            if (on[q]) yb[q] = load_local(ixp<true>(z, cc[q]));
         await_rows<T, CH>(z, cc, on, yb, err);
 #pragma unroll
         for (int q = 0; q < CH; q++)
@@ -358,6 +354,212 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
     }
 }
 
+// ------------------------------------------------------------------ BCSR, colored
+// One lane per row.  A wave takes bpw whole schedule blocks of bsize rows (bsize <= 64), or one
+// larger block in parts of at most 64 rows one after the other (a later part gathers the
+// earlier ones like any other row).  Per row, in the order of the sequential solve
+// (senk_sparse.hpp:399-415, 436-464): first the entries of BNL x BNW blocks outside the
+// part, in rounds of about 8 gathers, then the in-part columns step by step, each finished row
+// broadcast in the wave; the next in-part block's values are held in a short register queue.
+// Bound by the levels' chain (publish, poll, in-part steps).  Elasticity 45^3, blocks of 48, 11
+// colors, L + U in FP64: FIGURE us; one lane per schedule block walking its rows, one launch per
+// color (518 lanes in flight), 3196 us.
+template <typename T, int BNL, int BNW, bool UPPER>
+__global__ __launch_bounds__(64 * kCsrWaves) void k_bcsr_sweep(
+    SweepLevels lv, const int *__restrict__ blk_list, int bsize, int part, int bpw, const int *__restrict__ brptr,
+    const int *__restrict__ bcind, const T *__restrict__ bval, const T *x, T *y, T *z, T *reset, unsigned *err) {
+    using U = typename Bits<T>::U;
+    constexpr int BS = BNL * BNW, BREM = BNL / BNW;
+    constexpr int CB = BNW >= 8 ? 1 : (8 + BNW - 1) / BNW;  // blocks per round
+    constexpr int QB = BNW == 1 ? 8 : 4;                    // in-part blocks held in LDS
+    __shared__ int qc[kCsrWaves][QB][64];
+    __shared__ T qv[kCsrWaves][QB][BNW][64];
+    const int xs = (int)(blockIdx.x % kXcds), j = (int)(blockIdx.x / kXcds);
+    const int l = level_of(lv, j), sl = __builtin_amdgcn_readfirstlane(band_slice(lv, l, j, xs, bpw));
+    if (sl < 0) return;
+    const int lane = (int)(threadIdx.x & 63), wv = (int)(threadIdx.x >> 6);
+    const int nb = min(bpw, lv.units[l] - sl * bpw);  // blocks of this wave
+    const int slot = bpw > 1 ? lane / bsize : 0;
+    const bool has = slot < nb;
+    const int bu = lv.unit0[l] + sl * bpw + (has ? slot : 0);
+    const int blk = blk_list ? blk_list[bu] : bu;
+    const int nparts = (bsize + part - 1) / part;
+    for (int pq = 0; pq < nparts; pq++) {
+        const int p = UPPER ? nparts - 1 - pq : pq;
+        const int rows = min(part, bsize - p * part);
+        const int r = lane - slot * bsize;  // row in the part (bpw > 1: a whole block)
+        const bool active = has && r < rows;
+        const int base = blk * bsize + p * part, end = base + rows;
+        const int row = base + (active ? r : 0), g = row / BNL, kk = row % BNL;
+        const int lbase = slot * bsize;  // lane of the part's first row
+        T t = 0;
+        int first = 0, cnt = 0;          // the row's blocks outside its own diagonal (U), in solve order
+        T dg[BNL] = {};
+        if (active) {
+            t = x[row];
+            reset[row] = __builtin_bit_cast(T, Bits<T>::kSentinel);
+            const int b0 = brptr[g], b1 = brptr[g + 1];
+            if (UPPER) {
+                first = b1 - 1;
+                cnt = b1 - (b0 + BREM);
+#pragma unroll
+                for (int d = 0; d < BNL; d++)
+                    dg[d] = d >= kk ? bval[(size_t)(b0 + d / BNW) * BS + (d % BNW) * BNL + kk] : T(0);
+            } else {
+                first = b0;
+                cnt = b1 - b0;
+            }
+        }
+        auto at = [&](int i) { return UPPER ? first - i : first + i; };
+        // the place of the first in-part block, and whether the columns run strictly in solve order
+        int in0 = cnt, prev = UPPER ? 0x7fffffff : -1;
+        bool ordered = true;
+        for (int i0 = 0; __ballot(i0 < cnt); i0 += 8) {
+            int c[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (i0 + q < cnt) c[q] = bcind[at(i0 + q)] * BNW;
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (i0 + q < cnt) {
+                    ordered = ordered && (UPPER ? c[q] < prev : c[q] > prev);
+                    prev = c[q];
+                    if (UPPER ? c[q] < end : c[q] >= base) in0 = min(in0, i0 + q);
+                }
+        }
+        const bool slow = __ballot(!ordered) != 0;
+        const int outside = slow ? cnt : in0;  // blocks to look at for rows outside the part
+        // in-part columns: the lane's next QB blocks wait in LDS, requested before the wait below;
+        // the block after the current one is read ahead of its step
+        auto refill = [&](int i0) {
+            int c[QB];
+            T v[QB][BNW];
+#pragma unroll
+            for (int q = 0; q < QB; q++) {
+                c[q] = -1;
+                if (i0 + q < cnt) {
+                    const int b = at(i0 + q);
+                    c[q] = bcind[b] * BNW - base;
+                    const T *vb = bval + (size_t)b * BS + kk;
+#pragma unroll
+                    for (int m = 0; m < BNW; m++) v[q][m] = vb[m * BNL];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < QB; q++) {
+                qc[wv][q][lane] = c[q];
+#pragma unroll
+                for (int m = 0; m < BNW; m++)
+                    if (i0 + q < cnt) qv[wv][q][m][lane] = v[q][m];
+            }
+        };
+        refill(in0);
+        // outside the part
+        for (int i0 = 0; __ballot(i0 < outside); i0 += CB) {
+            int cc[CB * BNW];
+            bool on[CB * BNW];
+            T vv[CB * BNW];
+            U yb[CB * BNW];
+#pragma unroll
+            for (int q = 0; q < CB; q++) {
+                const bool have = i0 + q < outside;
+                const int c = have ? bcind[at(i0 + q)] * BNW : 0;
+                const bool out = have && (UPPER ? c >= end : c < base);
+#pragma unroll
+                for (int m = 0; m < BNW; m++) {
+                    cc[q * BNW + m] = c + m;
+                    on[q * BNW + m] = out;
+                    if (out) vv[q * BNW + m] = (bval + (size_t)at(i0 + q) * BS + kk)[m * BNL];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < CB * BNW; q++)
+                if (on[q]) yb[q] = load_local(ixp<true>(z, cc[q]));
+            await_rows<T, CB * BNW>(z, cc, on, yb, err);
+#pragma unroll
+            for (int q = 0; q < CB * BNW; q++)
+                if (on[q]) t -= vv[q] * __builtin_bit_cast(T, yb[q]);
+        }
+        auto bcast = [&](int i) {  // row i of every block's part
+            if (bpw == 1) {
+                if constexpr (sizeof(T) == 4) {
+                    return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t), i));
+                } else {
+                    const unsigned long long u = __builtin_bit_cast(unsigned long long, t);
+                    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, i);
+                    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), i);
+                    return __builtin_bit_cast(T, ((unsigned long long)hi << 32) | lo);
+                }
+            }
+            return __shfl(t, (lbase + i) & 63, 64);
+        };
+        int nq = 0, nc = -1;
+        T nv[BNW];
+        auto next = [&]() {
+            nc = qc[wv][nq][lane];
+#pragma unroll
+            for (int m = 0; m < BNW; m++) nv[m] = qv[wv][nq][m][lane];
+        };
+        next();
+        // The rows that hold the column block at c0 subtract it; value(m): column c0 + m.  A
+        // block of L may lie in its rows' own group, where column m is final only once the
+        // columns before it are subtracted: value(m) is asked for in that order.
+        auto take = [&](int c0, auto &&value) {
+            if (slow) {  // columns not in order: every block of the row is looked at
+                for (int m = 0; m < BNW; m++) {
+                    const T yc = value(m);
+                    for (int i = 0; i < cnt; i++) {
+                        const int b = at(i);
+                        if (bcind[b] * BNW - base == c0) t -= bval[(size_t)b * BS + m * BNL + kk] * yc;
+                    }
+                }
+                return;
+            }
+            const bool mine = nc == c0;
+            if (!__ballot(mine)) return;
+#pragma unroll
+            for (int m = 0; m < BNW; m++) {
+                const T yc = value(m);
+                if (mine) t -= nv[m] * yc;
+            }
+            if (mine) {
+                if (++nq == QB) {
+                    in0 += QB;
+                    refill(in0);
+                    nq = 0;
+                }
+                next();
+            }
+        };
+        if (!UPPER) {
+            for (int c0 = 0; c0 < rows; c0 += BNW) take(c0, [&](int m) { return bcast(c0 + m); });
+        } else {
+            for (int g0 = rows - BNL; g0 >= 0; g0 -= BNL) {
+                // the group's own triangle, its diagonal inverted
+                T yd[BNL];
+#pragma unroll
+                for (int d = BNL - 1; d >= 0; d--) {
+                    if (r == g0 + d) t = t * dg[d];
+                    yd[d] = bcast(g0 + d);
+                    if (r >= g0 && r < g0 + d) t -= dg[d] * yd[d];
+                }
+#pragma unroll
+                for (int q = BREM - 1; q >= 0; q--)
+                    take(g0 + q * BNW, [&](int m) {
+                        T v = yd[q * BNW];
+#pragma unroll
+                        for (int w = 1; w < BNW; w++) v = m == w ? yd[q * BNW + w] : v;
+                        return v;
+                    });
+            }
+        }
+        if (active) {
+            store_agent(z + row, canonical(t));
+            y[row] = t;
+        }
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_fill_sentinel2(size_t n, T *p) {
     for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
@@ -374,7 +576,7 @@ static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
     SweepVec *v = c->sweep;
     *ok = false;
     const size_t bytes = n * sizeof(T);
-    if (!c->sweep_err) return SENK_OK;
+    if (!c->sweep_err || bytes >= (size_t)1 << 32) return SENK_OK;  // z is addressed by 32-bit offsets
     if (v[0].bytes < bytes) {
         // grown while nothing of this context runs on it; allowed during a stream capture
         // of the calling thread (the context's stream is never captured)
@@ -429,27 +631,33 @@ static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
 // 203, 40^3 (542) 315 / 350, 61x64x67 (1377) 637 / 581; 27-point 38^3 (209) 1341 / 1437.
 constexpr double kPlanOneStream = 800;
 void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, int *streams, int *waves,
-                    std::vector<int> &seq, std::vector<int> &pos) {
-    const int S = s.nlev > 0 && (double)blk.size() / s.nlev < kPlanOneStream ? 1 : kXcds;
-    std::vector<int> of[kXcds];
-    for (int step = 0; step < s.nlev; step++) {
-        const int l = upper ? s.nlev - 1 - step : step;
-        const long long a = s.lev_ptr[l], n = s.lev_ptr[l + 1] - a;
-        for (int x = 0; x < S; x++)
-            of[x].insert(of[x].end(), blk.begin() + (a + n * x / S), blk.begin() + (a + n * (x + 1) / S));
+                    std::vector<int> &out) {
+    const size_t n = blk.size();
+    const int S = s.nlev > 0 && (double)n / s.nlev < kPlanOneStream ? 1 : kXcds;
+    size_t len[kXcds] = {};
+    for (int l = 0; l < s.nlev; l++) {
+        const long long k = s.lev_ptr[l + 1] - s.lev_ptr[l];
+        for (int x = 0; x < S; x++) len[x] += (size_t)(k * (x + 1) / S - k * x / S);
     }
     size_t w = 0;
-    for (int x = 0; x < S; x++) w = std::max(w, (of[x].size() + 63) / 64);
-    seq.assign(w * S * 64, -1);
-    pos.assign(blk.size(), 0);
-    for (int x = 0; x < S; x++)
-        for (size_t i = 0; i < of[x].size(); i++) {
-            const size_t p = ((i / 64) * S + x) * 64 + i % 64;
-            seq[p] = of[x][i];
-            pos[of[x][i]] = (int)p;
-        }
+    for (int x = 0; x < S; x++) w = std::max(w, (len[x] + 63) / 64);
     *streams = S;
     *waves = (int)w;
+    // blk, then the sequence, then each row's place in it
+    out.assign(n + w * S * 64 + n, -1);
+    std::copy(blk.begin(), blk.end(), out.begin());
+    int *seq = out.data() + n, *pos = seq + w * S * 64;
+    size_t at[kXcds] = {};
+    for (int step = 0; step < s.nlev; step++) {
+        const int l = upper ? s.nlev - 1 - step : step;
+        const long long a = s.lev_ptr[l], k = s.lev_ptr[l + 1] - a;
+        for (int x = 0; x < S; x++)
+            for (long long i = a + k * x / S; i < a + k * (x + 1) / S; i++) {
+                const size_t q = at[x]++, p = ((q / 64) * S + x) * 64 + q % 64;
+                seq[p] = blk[i];
+                pos[blk[i]] = (int)p;
+            }
+    }
 }
 
 // The level table of a schedule in solve order; units of a level: rows or blocks, `per` of
@@ -482,7 +690,7 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
                      const T *x, T *y, const double *in_scale, const int *stop, bool *done) {
     *done = false;
     const int BS = s.bsize;
-    if (BS < 1 || BS > 64 || 64 % BS || s.lev_ptr.empty() || s.lev_ptr[0] != 0 ||
+    if (N <= 0 || BS < 1 || BS > 64 || 64 % BS || s.lev_ptr.empty() || s.lev_ptr[0] != 0 ||
         (long long)s.lev_ptr[s.nlev] * BS != N)
         return SENK_OK;
     T *z = nullptr, *reset = nullptr;
@@ -542,5 +750,59 @@ template int launch_csr_sweep<double>(Ctx *, const Schedule &, bool, int, const 
                                       const double *, double *, const double *, const int *, bool *);
 template int launch_csr_sweep<float>(Ctx *, const Schedule &, bool, int, const int *, const int *, const float *,
                                      const float *, float *, const double *, const int *, bool *);
+
+template <typename T, int BNL, int BNW>
+static void bcsr_sweep(Ctx *c, const SweepLevels &lv, int tickets, const Schedule &s, bool upper, int part, int bpw,
+                       const int *brptr, const int *bcind, const T *bval, const T *x, T *y, T *z, T *reset) {
+    const int grid = kXcds * tickets;
+    if (upper)
+        k_bcsr_sweep<T, BNL, BNW, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, c->sweep_err_d);
+    else
+        k_bcsr_sweep<T, BNL, BNW, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, c->sweep_err_d);
+}
+template <typename T>
+int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,
+                      const int *bcind, const T *bval, const T *x, T *y, bool *done) {
+    *done = false;
+    if (bnl < 1 || bnw < 1 || bnl % bnw || s.bsize % bnl || s.lev_ptr.empty() || s.lev_ptr[0] != 0 ||
+        (long long)s.lev_ptr[s.nlev] * s.bsize != N)
+        return SENK_OK;
+    const int part = s.bsize <= 64 ? s.bsize : 64 / bnl * bnl;
+    const int bpw = s.bsize <= 64 ? 64 / s.bsize : 1;
+    SweepLevels lv;
+    int tickets = 0;
+    if (!sweep_levels(s, upper, 1, bpw, &lv, &tickets)) return SENK_OK;
+    T *z = nullptr, *reset = nullptr;
+    bool ok = false;
+    SENK_TRY(sweep_vectors<T>(c, (size_t)N, &z, &reset, &ok));
+    if (!ok) return SENK_OK;
+#define SENK_BCSR_SWEEP(A, B) \
+    case 16 * A + B: bcsr_sweep<T, A, B>(c, lv, tickets, s, upper, part, bpw, brptr, bcind, bval, x, y, z, reset); break
+    switch (16 * bnl + bnw) {
+        SENK_BCSR_SWEEP(1, 1);
+        SENK_BCSR_SWEEP(2, 1);
+        SENK_BCSR_SWEEP(2, 2);
+        SENK_BCSR_SWEEP(3, 1);
+        SENK_BCSR_SWEEP(3, 3);
+        SENK_BCSR_SWEEP(4, 1);
+        SENK_BCSR_SWEEP(4, 2);
+        SENK_BCSR_SWEEP(4, 4);
+        SENK_BCSR_SWEEP(8, 1);
+        SENK_BCSR_SWEEP(8, 2);
+        SENK_BCSR_SWEEP(8, 4);
+        SENK_BCSR_SWEEP(8, 8);
+        default: return SENK_ERR_UNSUPPORTED;  // as the launch per level
+    }
+#undef SENK_BCSR_SWEEP
+    SENK_LAUNCH_CHECK();
+    *done = true;
+    return SENK_OK;
+}
+template int launch_bcsr_sweep<double>(Ctx *, const Schedule &, bool, int, int, int, const int *, const int *,
+                                       const double *, const double *, double *, bool *);
+template int launch_bcsr_sweep<float>(Ctx *, const Schedule &, bool, int, int, int, const int *, const int *,
+                                      const float *, const float *, float *, bool *);
 
 }  // namespace senk_amd

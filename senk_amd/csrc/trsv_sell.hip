@@ -203,19 +203,6 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill(int nslices, const int4 *__
     if (UPPER) dinv[slot] = lr.active ? (DiagT<V>)val[s] : DiagT<V>(0);
 }
 
-// p + i; with O32 addressed as p's (uniform) base plus a 32-bit byte offset, one address
-// register per access instead of a 64-bit pair (the launch checks that every array of the
-// layout and every vector fits: i * sizeof(P) < 2^32)
-template <bool O32, typename P>
-__device__ __forceinline__ P *ixp(P *p, size_t i) {
-    if constexpr (O32) {
-        using Ch = typename std::conditional<std::is_const<P>::value, const char, char>::type;
-        return reinterpret_cast<P *>(reinterpret_cast<Ch *>(p) + (size_t)((unsigned)i * (unsigned)sizeof(P)));
-    } else {
-        return p + i;
-    }
-}
-
 // Sweep words (unsigned, device): the time-out flag and the ticket counter of mode 2.
 constexpr int kSweepErr = 0, kSweepTicket = 1, kSweepWords = 32;
 // workgroup size (waves = slices per ticket) of the per-XCD ticket streams: 8-wave

@@ -1,4 +1,5 @@
-"""Single-launch triangular solves on the caller's CSR factors (ABMC colors and plans).
+"""Single-launch triangular solves on the caller's CSR and BCSR factors (ABMC colors and
+plans).
 
 Every row keeps the sequential solve's operations and their order, so the results must be the
 oracle's sequential solve bit for bit, whatever solves of other sizes and types ran before
@@ -11,7 +12,7 @@ import pytest
 
 import senk_amd as S
 from oracle import oracle as O
-from tests.helpers import abmc_system, ilu_factors
+from tests.helpers import abmc_system, ilu_factors, oracle_ilu0, relerr
 
 pytestmark = pytest.mark.gpu
 
@@ -96,6 +97,10 @@ def test_plans_in_turn_with_other_sizes(ctx, dt):
     other = np.float32 if dt == np.float64 else np.float64
     _plan_case(ctx, S.gen_poisson7(13, 9, 11), dt)        # one stream
     _plan_case(ctx, _tridiagonal(1), other)
+    empty = C.c_void_p()
+    S.call("senk_trsv_plan_create", ctx.h, O.P(np.zeros(1, np.int32)), O.P(np.zeros(1, np.int32)), 0, 0, C.byref(empty))
+    S.call("senk_sptrsv_csr_l_f64", ctx.h, empty, None, None, None, None, None, 0)
+    S.lib().senk_trsv_plan_destroy(empty)
     _plan_case(ctx, _tridiagonal(333), dt)                # every row waits on one of its own wave
     _plan_case(ctx, S.gen_convdiff27(12, 10.0), dt)       # rows of 13
     _plan_case(ctx, S.gen_unstructured(20000, 7), dt)     # long rows, several rounds
@@ -143,3 +148,48 @@ def test_schedules_outside_the_single_launch(ctx):
     S.call("senk_sptrsv_csr_l_amc_f64", ctx.h, *(t.p for t in d[:3]), d[6].p, dy2.p, N, O.P(part), 200)
     out = dy2.download()
     assert np.array_equal(out[:200], yl[:200]) and np.all(out[200:] == 7.0)
+
+
+def _bcsr(ctx, n, bnl, bnw, bsize, shuffle=False):
+    """(device result of L, of U, oracle's of L, of U) on an elasticity (bnl 3) or 27-point system."""
+    mat = S.gen_elasticity3(n, 2) if bnl == 3 else S.gen_convdiff27(n, 10.0)
+    val, cind, rptr, N = S.padding(mat[2], mat[1], mat[0], bsize, len(mat[0]) - 1)
+    sy = abmc_system(rptr, cind, val, bsize)
+    fv, fc, fr = S.alloc_block_zero(sy["val"], sy["cind"], sy["rptr"], N, bnl, bnw)
+    sp = S.split(oracle_ilu0(fv, fc, fr), fc, fr, N, "L-DU", True)
+    bl, bu = S.csr2bcsr(*sp["L"], N, bnl, bnw), S.csr2bcsr(*sp["U"], N, bnl, bnw)
+    x = np.random.default_rng(10).uniform(-1, 1, N)
+    yl, yu = np.zeros(N), np.zeros(N)
+    tail = (N, O.P(sy["cptr"]), sy["nc"], bsize, bnl, bnw)
+    O.orc().or_sptrsv_bcsr_l_abmc_d(*(O.P(t) for t in bl), O.P(x), O.P(yl), *tail)
+    O.orc().or_sptrsv_bcsr_u_abmc_d(*(O.P(t) for t in bu), O.P(yl), O.P(yu), *tail)
+    if shuffle:  # the blocks of every row in another order (U keeps its diagonal ones first)
+        rng, bs = np.random.default_rng(1), bnl * bnw
+        for v, c, r, keep in ((*bl, 0), (*bu, bnl // bnw)):
+            for g in range(N // bnl):
+                k = np.arange(r[g] + keep, r[g + 1])
+                o = rng.permutation(k)
+                c[k], v.reshape(-1, bs)[k] = c[o].copy(), v.reshape(-1, bs)[o].copy()
+    d = [ctx.array(t) for t in (*bl, *bu, x)]
+    dy = ctx.zeros(N)
+    S.call("senk_sptrsv_bcsr_l_abmc_f64", ctx.h, *(t.p for t in d[:3]), d[6].p, dy.p, *tail)
+    t = dy.download()
+    S.call("senk_sptrsv_bcsr_u_abmc_f64", ctx.h, *(t.p for t in d[3:6]), dy.p, dy.p, *tail)
+    return t, dy.download(), yl, yu
+
+
+# several blocks a wave, one, and blocks of more rows than a wave (in parts); every block shape
+@pytest.mark.parametrize("bnl,bnw,bsize", [(1, 1, 5), (2, 1, 6), (2, 2, 64), (3, 1, 24), (3, 3, 24), (3, 3, 48),
+                                           (3, 3, 63), (3, 3, 96), (4, 1, 20), (4, 2, 40), (4, 4, 128), (8, 1, 16),
+                                           (8, 2, 8), (8, 4, 72), (8, 8, 64)])
+def test_bcsr_abmc_bitwise(ctx, bnl, bnw, bsize):
+    t, u, yl, yu = _bcsr(ctx, 9, bnl, bnw, bsize)
+    assert np.array_equal(t, yl) and np.array_equal(u, yu)
+
+
+@pytest.mark.parametrize("bnl,bnw,bsize", [(3, 3, 48), (2, 1, 8), (4, 4, 96)])
+def test_bcsr_blocks_in_any_order(ctx, bnl, bnw, bsize):
+    """Blocks of a row out of order: the same sums in another order (rows of at most 27 blocks,
+    so a few tens of roundings each)."""
+    t, u, yl, yu = _bcsr(ctx, 8, bnl, bnw, bsize, shuffle=True)
+    assert relerr(t, yl) <= 1e-13 and relerr(u, yu) <= 1e-13
