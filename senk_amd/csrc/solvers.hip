@@ -309,6 +309,127 @@ __global__ __launch_bounds__(kBlock) void k_mgs(int N, int k, int j, const T *__
     store_partials<1>(v, Pout);
 }
 
+// Modified Gram-Schmidt of w against V_0..V_{K-1} (K = j+1 <= kMgsMaxK) with two passes over
+// the basis instead of one launch per column.  With q_k = sig_k V_k the coefficients that the
+// column-by-column subtraction produces satisfy (I + L) h = Q^T w, L the strictly lower part
+// of Q^T Q, so h = T Q^T w with T = (I + L)^-1 (the compact form of modified Gram-Schmidt,
+// Swirydowicz, Langou, Ananthan, Yang and Thomas 2021).  T grows by one row per iteration:
+// row j = -(q_j^T q_i)_{i<j} T, its inner products formed in the same pass as Q^T w.
+//   k_mgs_dots    partials of (V_k, w) and (V_k, V_j)
+//   k_mgs_fin     the sums, scaled (one workgroup per product)
+//   k_mgs_update  T's new row, h, w -= V h, partials of (w, w)
+// Reads of the basis per iteration: 2 K vectors and 3 launches, where a launch per column
+// reads and writes 4 K in K + 1 launches.  GMRES(30), 64^3 variable-coefficient system
+// (vectors of 2 MB, bound by the launches): 36.2 -> 25.8 ms for 281 iterations; 128^3 (16.8 MB,
+// bound by the bytes): 257.9 -> 197.6 ms for 566.
+constexpr int kMgsMaxK = 64;  // longer recurrences (m > 64) take the launch per column
+constexpr int kMgsChunk = 32; // columns per k_mgs_dots launch (its accumulators)
+template <typename T, int KMAX>
+__global__ __launch_bounds__(kBlock) void k_mgs_dots(int N, int K, const T *__restrict__ V, size_t ld,
+                                                     const T *__restrict__ w, const T *__restrict__ vj,
+                                                     double *Pw, double *Pg, const int *stop) {
+    if (*stop) return;
+    double aw[KMAX], ag[KMAX];
+#pragma unroll
+    for (int k = 0; k < KMAX; k++) aw[k] = ag[k] = 0;
+    SENK_FOR4(i0, N) {
+        T wv[4], jv[4];
+        get4(w, i0, N, wv);
+        get4(vj, i0, N, jv);
+#pragma unroll
+        for (int k = 0; k < KMAX; k++)
+            if (k < K) {
+                T vk[4];
+                get4(V + (size_t)k * ld, i0, N, vk);
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    aw[k] += (double)vk[u] * (double)wv[u];
+                    ag[k] += (double)vk[u] * (double)jv[u];
+                }
+            }
+    }
+    store_partials_n<KMAX>(aw, K, Pw);
+    store_partials_n<KMAX>(ag, K, Pg);
+}
+// dw[k] = sig_k (V_k, w), dg[k] = sig_k sig_j (V_k, V_j): workgroups [0, K) and [K, 2K)
+__global__ __launch_bounds__(kBlock) void k_mgs_fin(const double *Pw, const double *Pg, int K, int B,
+                                                    const double *sig, const double *sigj, double *dw, double *dg,
+                                                    const int *stop) {
+    if (*stop) return;
+    const int k = (int)blockIdx.x % K;
+    const bool gram = (int)blockIdx.x >= K;
+    const double s = sum_partials((gram ? Pg : Pw) + (size_t)k * kPartLd, B);
+    if (threadIdx.x != 0) return;
+    if (gram) dg[k] = sig[k] * *sigj * s;
+    else dw[k] = sig[k] * s;
+}
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_mgs_update(int N, int j, const T *__restrict__ V, size_t ld,
+                                                       const double *sig, const double *dw, const double *dg,
+                                                       double *Tm, double *hc, T *w, double *Pout,
+                                                       const int *stop) {
+    if (*stop) return;
+    __shared__ double tm[kMgsMaxK][kMgsMaxK + 1], rw[kMgsMaxK], rg[kMgsMaxK], cf[kMgsMaxK];
+    const int K = j + 1;
+    for (int e = threadIdx.x; e < j * j; e += kBlock) tm[e / j][e % j] = Tm[(size_t)(e / j) * kMgsMaxK + e % j];
+    if (threadIdx.x < K) {
+        rw[threadIdx.x] = dw[threadIdx.x];
+        rg[threadIdx.x] = dg[threadIdx.x];
+    }
+    __syncthreads();
+    // row j of T (lower triangular with a unit diagonal: nothing above it is read)
+    const int t = threadIdx.x;
+    if (t < K) {
+        double a = t == j ? 1.0 : 0.0;
+        for (int i = t; i < j; i++) a -= rg[i] * tm[i][t];
+        tm[j][t] = a;
+        if (blockIdx.x == 0) Tm[(size_t)j * kMgsMaxK + t] = a;
+    }
+    __syncthreads();
+    if (t < K) {
+        double h = 0;
+        for (int k = 0; k <= t; k++) h += tm[t][k] * rw[k];
+        cf[t] = h * sig[t];
+        if (blockIdx.x == 0) hc[t] = h;
+    }
+    __syncthreads();
+    double acc = 0;
+    SENK_FOR4(i0, N) {
+        T wv[4];
+        double sv[4];
+        get4(w, i0, N, wv);
+#pragma unroll
+        for (int u = 0; u < 4; u++) sv[u] = (double)wv[u];
+#pragma unroll 4
+        for (int k = 0; k < K; k++) {
+            T vk[4];
+            get4(V + (size_t)k * ld, i0, N, vk);
+#pragma unroll
+            for (int u = 0; u < 4; u++) sv[u] -= cf[k] * (double)vk[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            wv[u] = (T)sv[u];
+            acc += (double)wv[u] * (double)wv[u];
+        }
+        put4(w, i0, N, wv);
+    }
+    const double v[1] = {acc};
+    store_partials<1>(v, Pout);
+}
+template <typename T>
+void launch_mgs_dots(Ctx *c, int B, int N, int K, const T *V, size_t ld, const T *w, const T *vj, double *Pw,
+                     double *Pg, const int *stop) {
+    if (K <= 8)
+        k_mgs_dots<T, 8><<<B, kBlock, 0, c->stream>>>(N, K, V, ld, w, vj, Pw, Pg, stop);
+    else if (K <= 16)
+        k_mgs_dots<T, 16><<<B, kBlock, 0, c->stream>>>(N, K, V, ld, w, vj, Pw, Pg, stop);
+    else if (K <= 24)
+        k_mgs_dots<T, 24><<<B, kBlock, 0, c->stream>>>(N, K, V, ld, w, vj, Pw, Pg, stop);
+    else
+        k_mgs_dots<T, kMgsChunk><<<B, kBlock, 0, c->stream>>>(N, K, V, ld, w, vj, Pw, Pg, stop);
+}
+
 // Classical Gram-Schmidt with re-orthogonalisation (CGS2), one pass over V_0..V_{K-1}
 // (K = j+1 <= kRedMaxK):
 //   coef != nullptr:  w -= sum_k coef[k]*sig[k] V_k  first
@@ -394,37 +515,58 @@ __global__ __launch_bounds__(kBlock) void k_gmres_tail(int j, int m, double *H, 
         if (mark && threadIdx.x == 0) write_mark(mark, seq, 1);
         return;
     }
-    const double nn = sum_partials(Pn, B);
-    if (threadIdx.x != 0) return;
+    // the column and the rotations in LDS first: the chain below then waits for no memory
+    __shared__ double col[kMgsMaxK + 1], c_[kMgsMaxK + 1], s_[kMgsMaxK + 1];
     double *hc = H + (size_t)j * (m + 1);
-    if (add_h)
-        for (int k = 0; k <= j; k++) hc[k] += add_h[k];
-    const double hn = sqrt(nn);
-    hc[j + 1] = hn;
-    sig[j + 1] = 1.0 / hn;
-    for (int k = 0; k < j; k++) {
-        const double a = hc[k], b = hc[k + 1];
-        hc[k] = cs[k] * a - sn[k] * b;
-        hc[k + 1] = sn[k] * a + cs[k] * b;
+    const bool staged = j <= kMgsMaxK;
+    if (staged && threadIdx.x <= j) {
+        col[threadIdx.x] = hc[threadIdx.x] + (add_h ? add_h[threadIdx.x] : 0.0);
+        c_[threadIdx.x] = cs[threadIdx.x];
+        s_[threadIdx.x] = sn[threadIdx.x];
     }
-    const double a = hc[j], b = hc[j + 1];
-    const double r = sqrt(a * a + b * b);
-    cs[j] = a / r;
-    sn[j] = -b / r;
+    const double ej = e[j];
+    const double nn = sum_partials(Pn, B);  // a barrier on the way
+    if (threadIdx.x >= 64) return;
+    const double hn = sqrt(nn);
+    double a;
+    if (staged) {
+        a = col[0];
+        for (int k = 0; k < j; k++) {
+            const double b = col[k + 1], ck = c_[k], sk = s_[k];
+            if ((int)threadIdx.x == k) hc[k] = ck * a - sk * b;
+            a = sk * a + ck * b;
+        }
+    } else {
+        if (threadIdx.x != 0) return;
+        a = hc[0] + (add_h ? add_h[0] : 0.0);
+        for (int k = 0; k < j; k++) {
+            const double b = hc[k + 1] + (add_h ? add_h[k + 1] : 0.0);
+            hc[k] = cs[k] * a - sn[k] * b;
+            a = sn[k] * a + cs[k] * b;
+        }
+    }
+    if (threadIdx.x != 0) return;
+    sig[j + 1] = 1.0 / hn;
+    const double r = sqrt(a * a + hn * hn);
+    const double cj = a / r, sj = -hn / r, en = sj * ej;
+    cs[j] = cj;
+    sn[j] = sj;
     hc[j] = r;
     hc[j + 1] = 0;
-    e[j + 1] = sn[j] * e[j];
-    e[j] = cs[j] * e[j];
-    const double ae = fabs(e[j + 1]);
+    e[j + 1] = en;
+    e[j] = cj * ej;
+    const double ae = fabs(en);
     if (hist && hidx < hcap) hist[hidx] = ae / nrm_b;
     state[1] = j + 1;
+    int stopped = 0;
     if (!isfinite(ae) || !isfinite(r)) {
         state[2] = 1;
-        state[0] = 1;
+        stopped = 1;
     } else if (ae <= tol) {
-        state[0] = 1;
+        stopped = 1;
     }
-    if (mark) write_mark(mark, seq, state[0]);
+    if (stopped) state[0] = 1;
+    if (mark) write_mark(mark, seq, stopped);
 }
 
 // Cycle end: y = Trsv(H, e) over the jdone columns (senk_blas2.hpp:24-34) and the
@@ -587,7 +729,8 @@ static int gmres(Ctx *c, const MatView &A, const PrecView &M, const T *b, T *x, 
     const int hcap = p.outer * m;
     size_t need = bytes_of<T>((size_t)(m + 1) * ld) + (flexible ? bytes_of<T>((size_t)m * ld) : 0) +
                   3 * bytes_of<T>(N) + bytes_of<double>((size_t)(m + 1) * m) + 7 * bytes_of<double>(m + 2) +
-                  bytes_of<double>(hcap + 1) + bytes_of<int>(8);
+                  bytes_of<double>(hcap + 1) + bytes_of<int>(8) + bytes_of<double>(kMgsMaxK * kMgsMaxK) +
+                  2 * bytes_of<double>(kMgsMaxK);
     void *wsp;
     SENK_TRY(ctx_work(c, need, &wsp));
     Carver cv{(char *)wsp, 0, need};
@@ -600,6 +743,8 @@ static int gmres(Ctx *c, const MatView &A, const PrecView &M, const T *b, T *x, 
     double *h2 = cv.take<double>(m + 2);
     double *dhist = cv.take<double>(hcap + 1);
     int *state = cv.take<int>(8);
+    double *Tm = cv.take<double>(kMgsMaxK * kMgsMaxK);  // modified Gram-Schmidt: T, Q^T w, Q^T q_j
+    double *mw = cv.take<double>(kMgsMaxK), *mg = cv.take<double>(kMgsMaxK);
 
     Poller poll;
     SENK_TRY(poll.init(c, state));
@@ -647,6 +792,21 @@ static int gmres(Ctx *c, const MatView &A, const PrecView &M, const T *b, T *x, 
                 SENK_LAUNCH_CHECK();
                 Pnorm = red_slot(c, kSlotC);
                 add_h = h2;
+            } else if (m <= kMgsMaxK) {
+                const int K = j + 1;
+                for (int k0 = 0; k0 < K; k0 += kMgsChunk) {
+                    const int kc = std::min(kMgsChunk, K - k0);
+                    launch_mgs_dots<T>(c, B, N, kc, V + (size_t)k0 * ld, ld, w, vj, red_slot(c, kSlotMgsA),
+                                       red_slot(c, kSlotMgsB), state);
+                    SENK_LAUNCH_CHECK();
+                    k_mgs_fin<<<2 * kc, kBlock, 0, c->stream>>>(red_slot(c, kSlotMgsA), red_slot(c, kSlotMgsB), kc, B,
+                                                                sig + k0, sig + j, mw + k0, mg + k0, state);
+                    SENK_LAUNCH_CHECK();
+                }
+                k_mgs_update<T><<<B, kBlock, 0, c->stream>>>(N, j, V, ld, sig, mw, mg, Tm, hc, w,
+                                                             red_slot(c, kSlotC), state);
+                SENK_LAUNCH_CHECK();
+                Pnorm = red_slot(c, kSlotC);
             } else {
                 for (int k = 0; k <= j + 1; k++) {
                     const double *Pin = red_slot(c, (k + 1) % 2 ? kSlotMgsB : kSlotMgsA);
