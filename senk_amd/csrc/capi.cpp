@@ -845,18 +845,20 @@ static int ilu0_impl(senk_ctx ctx, T *dval, const int *dcind, const int *drptr, 
         s.nlev = host::levels(hrptr, hcind, N, 1, false, s.lev_ptr, blk);
         SENK_TRY(upload(ctx, &s.dblk, blk.data(), blk.size()));
     }
-    int *dpos = nullptr, *derr = nullptr;
-    SENK_TRY(dalloc(&dpos, (size_t)N));
-    SENK_TRY(dalloc(&derr, 1));
-    SENK_HIP(hipMemsetAsync(derr, 0, sizeof(int), c->stream));
-    SENK_TRY(launch_find_diag(c, N, drptr, dcind, dpos));
-    SENK_TRY(launch_ilu0<T>(c, s, N, drptr, dcind, dpos, dval, derr));
-    int herr = 0;
-    SENK_HIP(hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SENK_HIP(hipStreamSynchronize(c->stream));
-    (void)hipFree(dpos);
-    (void)hipFree(derr);
+    // diagonal positions and the error word in the context's arena
+    void *buf = nullptr;
+    int st = ctx_work(c, ((size_t)N + 1) * sizeof(int), &buf);
+    int *dpos = static_cast<int *>(buf), *derr = dpos + N;
+    if (!st && hipMemsetAsync(derr, 0, sizeof(int), c->stream) != hipSuccess) st = SENK_ERR_HIP;
+    if (!st) st = launch_find_diag(c, N, drptr, dcind, dpos);
+    if (!st) st = launch_ilu0<T>(c, s, N, drptr, dcind, dpos, dval, derr);
+    int *herr_p = c->hpinned_i + 2;
+    if (!st && hipMemcpyAsync(herr_p, derr, sizeof(int), hipMemcpyDeviceToHost, c->stream) != hipSuccess)
+        st = SENK_ERR_HIP;
+    if (hipStreamSynchronize(c->stream) != hipSuccess && !st) st = SENK_ERR_HIP;
     if (s.dblk) (void)hipFree(s.dblk);
+    if (st) return st;
+    const int herr = *herr_p;
     if (herr == 1) return SENK_ERR_ZERO_PIVOT;
     if (herr == 2) return SENK_ERR_UNSUPPORTED;
     return SENK_OK;

@@ -1,0 +1,69 @@
+"""The grouped ILU(0) kernel (several lanes per row, rows in LDS) against the oracle's Ilu0.
+
+Same operations per entry in the same order: the same bits in FP64 and FP32, for every block
+size it takes, rows around its two group widths, and the cases it hands on."""
+import numpy as np
+import pytest
+
+import senk_amd as S
+from oracle import oracle as O
+from tests.helpers import abmc_system
+
+pytestmark = pytest.mark.gpu
+
+
+def _factor(ctx, val, cind, rptr, N, dt, cptr=None, nc=0, bsize=1):
+    v = np.ascontiguousarray(val.astype(dt))
+    fo = v.copy()
+    assert getattr(O.orc(), "or_ilu0_d" if dt == np.float64 else "or_ilu0_f")(O.P(fo), O.P(cind), O.P(rptr), N) == 0
+    d = [ctx.array(t) for t in (v, cind, rptr)]
+    S.call("senk_ilu0_f64" if dt == np.float64 else "senk_ilu0_f32", ctx.h, *(t.p for t in d), N,
+           None if cptr is None else O.P(cptr), nc, bsize, O.P(rptr), O.P(cind))
+    return d[0].download(), fo
+
+
+@pytest.mark.parametrize("bsize", [1, 2, 4, 8, 16, 32, 64, 48])
+@pytest.mark.parametrize("gen", ["poisson7", "convdiff27", "unstructured"])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_colored_bitwise(ctx, bsize, gen, dt):
+    mat = {"poisson7": lambda: S.gen_poisson7(11, 9, 7), "convdiff27": lambda: S.gen_convdiff27(8, 10.0),
+           "unstructured": lambda: S.gen_unstructured(1500, 4)}[gen]()
+    val, cind, rptr, N = S.padding(mat[2], mat[1], mat[0], bsize, len(mat[0]) - 1)
+    sy = abmc_system(rptr, cind, val, bsize)
+    f, fo = _factor(ctx, sy["val"], sy["cind"], sy["rptr"], N, dt, sy["cptr"], sy["nc"], bsize)
+    assert np.array_equal(f, fo)
+
+
+# dependency levels (lists of rows); 16 and 17 entries a row, and rows whose workgroup exceeds
+# the LDS limit (the wave-per-block kernel)
+@pytest.mark.parametrize("width", [7, 16, 17, 90, 400])
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_levels_of_banded_rows_bitwise(ctx, width, dt):
+    rng, N, h = np.random.default_rng(width), 700, width // 2
+    rows = [np.unique(np.clip(np.concatenate([[i], i + rng.integers(-3 * h, 3 * h + 1, width - 1)]), 0, N - 1))
+            for i in range(N)]
+    rptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    cind = np.concatenate(rows).astype(np.int32)
+    val = rng.uniform(-1, 1, len(cind))
+    for i in range(N):
+        val[rptr[i] + np.searchsorted(rows[i], i)] = 2.0 + len(rows[i])
+    f, fo = _factor(ctx, val, cind, rptr, N, dt)
+    assert np.array_equal(f, fo)
+
+
+@pytest.mark.parametrize("where", ["block", "other"])
+def test_zero_pivot_inside_and_outside_the_block(ctx, where):
+    N, bs = 8, 4
+    A = np.eye(N) * 3
+    i, j = (1, 0) if where == "block" else (5, 2)
+    A[i, j], A[j, j] = 1.0, 0.0
+    rptr, cind, val = [0], [], []
+    for r in range(N):
+        for c in range(N):
+            if A[r, c] != 0 or r == c:
+                cind.append(c)
+                val.append(A[r, c])
+        rptr.append(len(cind))
+    d = [ctx.array(np.array(t, dt)) for t, dt in ((val, np.float64), (cind, np.int32), (rptr, np.int32))]
+    cptr = np.array([0, 1, 2], np.int32)
+    assert S.lib().senk_ilu0_f64(ctx.h, *(t.p for t in d), N, O.P(cptr), 2, bs, None, None) == 3
