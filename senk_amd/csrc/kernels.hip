@@ -9,10 +9,15 @@
 namespace senk_amd {
 
 // =============================================================== SpMV CSR
-// G lanes per row (G | 64).  Lane q of a row sums entries rptr[row]+q, +G, ... in
-// order; the G partial sums are then combined by a butterfly inside the lane group.
-// Rows are walked grid-stride so that the fused residual form can reduce ||y||^2
-// with a bounded grid.
+// A wave takes R consecutive rows.  Their entries are one run of the matrix arrays, read 512 at
+// a time with coalesced loads, eight entries per lane: columns and values first, then the
+// gathers of x, and the products go to LDS; 64 / R lanes per row then add the row's products.
+// The next 512 entries are requested before the products are added.  Bound by the matrix stream
+// on large systems and by the chain rows -> entries -> x on small ones.  Against a kernel with
+// 1 to 64 lanes per row, each striding through it, us in FP64 / FP32: 7-point 100^3 29.4 ->
+// 26.0 / 18.9 -> 14.9, 27-point 64^3 26.1 -> 24.2 / 21.0 -> 16.2, unstructured 400,000 rows 27.9
+// -> 24.4 / 22.1 -> 15.0.  Four consecutive entries per lane (16-byte loads of the matrix) were
+// slower, 33.2 / 21.7 at 7-point 100^3: a wave's gathers then touch more lines each.
 template <typename T, int G>
 __device__ __forceinline__ T group_sum(T v) {
 #pragma unroll
@@ -20,49 +25,76 @@ __device__ __forceinline__ T group_sum(T v) {
     return v;
 }
 
-template <typename T, int G>
+template <typename T, int R>
 __global__ __launch_bounds__(kBlock) void k_spmv_csr(int N, const int *__restrict__ rptr,
                                                      const int *__restrict__ cind, const T *__restrict__ val,
                                                      const T *__restrict__ x, T *__restrict__ y,
                                                      const int *__restrict__ stop) {
+    constexpr int P = 64 / R, U = 8, W = 64 * U;  // lanes per row, entries per lane and per window
+    __shared__ T prod[kWavesPerBlock][W];
     if (stop && *stop) return;
-    const long long gid = (long long)xcd_block() * kBlock + threadIdx.x;
-    const int row = (int)(gid / G), q = (int)(gid % G);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const long long first = ((long long)xcd_block() * kWavesPerBlock + wv) * R;
+    if (first >= N) return;
+    const int r0 = (int)first, nr = min(R, N - r0);
+    const int rp = rptr[r0 + min(lane, nr)];
+    const int e0 = __builtin_amdgcn_readfirstlane(rp);
+    const int e1 = R < 64 ? __shfl(rp, nr, 64) : rptr[r0 + nr];
+    const int lr = lane / P, sub = lane % P;
+    const int rs = __shfl(rp, min(lr, nr), 64);
+    const int nx = __shfl(rp, min(lr + 1, 63), 64);
+    const int re = lr + 1 < nr ? nx : e1;
     T acc = 0;
-    if (row < N) {
-        const int e = rptr[row + 1];
-        // chunks of 4 independent gathers per lane, summed in entry order
-        for (int j0 = rptr[row] + q; j0 < e; j0 += 4 * G) {
-            T xv[4], vv[4];
+    int c[U];
+    T v[U];
+    auto load = [&](int w0) {
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int j = j0 + u * G;
-                if (j < e) {
-                    vv[u] = val[j];
-                    xv[u] = x[cind[j]];
-                }
+        for (int u = 0; u < U; u++) {
+            const int o = lane + 64 * u;
+            if (o < e1 - w0) {
+                c[u] = cind[w0 + o];
+                v[u] = val[w0 + o];
             }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (j0 + u * G < e) acc += vv[u] * xv[u];
         }
+    };
+    load(e0);
+    for (int w0 = e0; w0 < e1;) {
+        const int n = min(W, e1 - w0);
+        T xv[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (lane + 64 * u < n) xv[u] = x[c[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (lane + 64 * u < n) prod[wv][lane + 64 * u] = v[u] * xv[u];
+        if (e1 - w0 > W) load(w0 + W);
+        wave_lds_sync();
+        if (lr < nr) {
+            const int a = max(rs - w0, 0), b = min(re - w0, n);
+            for (int j = a + sub; j < b; j += P) acc += prod[wv][j];
+        }
+        wave_lds_sync();
+        if (e1 - w0 <= W) break;
+        w0 += W;
     }
-    acc = group_sum<T, G>(acc);
-    if (q == 0 && row < N) y[row] = acc;
+    acc = group_sum<T, P>(acc);
+    if (sub == 0 && lr < nr) y[r0 + lr] = acc;
 }
 
 template <typename T>
 int launch_spmv_csr(Ctx *c, int N, const int *rptr, const int *cind, const T *val, const T *x, T *y,
                     double avg_row, const int *stop) {
     if (N <= 0) return SENK_OK;
-    int G = avg_row > 48 ? 64 : avg_row > 24 ? 16 : avg_row > 12 ? 8 : avg_row > 6 ? 4 : avg_row > 3 ? 2 : 1;
-    long long threads = (long long)N * G;
-    int grid = (int)((threads + kBlock - 1) / kBlock);
-    switch (G) {
+    // Rows per wave: at most about one window of entries; fewer where that leaves under 2048 waves
+    // (two per SIMD), but not under some 100 entries (27-point 30^3 in FP64: 5.9 us with 16 rows a
+    // wave, 1688 waves; 5.2 with 4, 108 entries each; unstructured 60,013 rows: 6.3 us with 16,
+    // 8.1 with 4, 60 entries each)
+    int R = 64;
+    while (R > 1 && (R * avg_row > 512 || (N / R < 2048 && R * avg_row >= 4 * 96))) R /= 4;
+    const int grid = (int)(((long long)N + (long long)R * kWavesPerBlock - 1) / ((long long)R * kWavesPerBlock));
+    switch (R) {
         case 1: k_spmv_csr<T, 1><<<grid, kBlock, 0, c->stream>>>(N, rptr, cind, val, x, y, stop); break;
-        case 2: k_spmv_csr<T, 2><<<grid, kBlock, 0, c->stream>>>(N, rptr, cind, val, x, y, stop); break;
         case 4: k_spmv_csr<T, 4><<<grid, kBlock, 0, c->stream>>>(N, rptr, cind, val, x, y, stop); break;
-        case 8: k_spmv_csr<T, 8><<<grid, kBlock, 0, c->stream>>>(N, rptr, cind, val, x, y, stop); break;
         case 16: k_spmv_csr<T, 16><<<grid, kBlock, 0, c->stream>>>(N, rptr, cind, val, x, y, stop); break;
         default: k_spmv_csr<T, 64><<<grid, kBlock, 0, c->stream>>>(N, rptr, cind, val, x, y, stop); break;
     }
