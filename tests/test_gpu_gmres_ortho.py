@@ -38,3 +38,26 @@ def test_residual_history_matches_the_oracle(ctx, m):
     big = ho > 1e-8 * ho[0]
     assert big.sum() >= min(30, len(ho))
     assert np.max(np.abs(hd[big] - ho[big]) / ho[big]) <= 1e-8
+
+
+# one lane per row of the cycle end's triangular solve up to 64 columns, several beyond
+@pytest.mark.parametrize("m", [1, 2, 63, 64, 65, 128, 129])
+def test_solution_of_one_cycle_matches_the_oracle(ctx, m):
+    # x = V y is the minimiser over the Krylov space: its error is a few roundings times the
+    # condition number (below 1e3 here), far below 1e-9 relative
+    rptr, cind, val = S.gen_convdiff27(20, 10.0)
+    N = len(rptr) - 1
+    x = S.gen_uniform(5, N)
+    b = np.zeros(N)
+    O.orc().or_spmv_csr_d(O.P(val), O.P(cind), O.P(rptr), O.P(x), O.P(b), N)
+    nrm_b, eps = float(np.linalg.norm(b)), 1e-30
+    ho, hd = np.zeros(m), np.zeros(m)
+    xo, conv = np.zeros(N), C.c_int()
+    spec = O.prec_spec(0)
+    O.orc().or_gmres_d(O.P(val), O.P(cind), O.P(rptr), C.byref(spec), O.P(b), O.P(xo), nrm_b, 1, m, N, eps,
+                       O.P(ho), len(ho), C.byref(conv))
+    dv, dc, dr, db, dx = ctx.array(val), ctx.array(cind), ctx.array(rptr), ctx.array(b), ctx.zeros(N)
+    res = S.senk_result()
+    S.call("senk_gmresm_f64", ctx.h, dv.p, dc.p, dr.p, db.p, dx.p, C.c_double(nrm_b), 1, m, N, C.c_double(eps), 0,
+           C.byref(res), O.P(hd), len(hd))
+    assert np.linalg.norm(dx.download() - xo) <= 1e-9 * np.linalg.norm(xo)
