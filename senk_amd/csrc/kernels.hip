@@ -733,11 +733,12 @@ template int launch_sptrsv_bcsr<float>(Ctx *, const Schedule &, bool, int, int, 
 // workgroup, the workgroup's rows (columns and values) in LDS.  Each pivot's upper entries
 // are spread over the row's lanes, which look their columns up among the row's later entries
 // (ascending, binary search in LDS) and update distinct entries.  First come the pivot rows
-// outside the block, final in memory, requested one pivot ahead; then BS - 1 steps inside the
+// outside the block, final in memory, their places requested two pivots ahead and their values
+// one; then BS - 1 steps inside the
 // block, step c eliminating with row c, final in LDS.  Bound by the chain of pivots of one row;
 // the rows of a color advance together, where the kernel below walks a block's rows one by
 // one with some six dependent loads per pivot.  Per call, FP64: 7-point 96^3, blocks of 8, 10
-// colors: 1577 -> 356 us; 27-point 48^3, blocks of 16, 13 colors: 6313 -> 810 us; with one
+// colors: 1577 -> 349 us; 27-point 48^3, blocks of 16, 13 colors: 6313 -> 789 us; with one
 // lane per row and a serial merge 382 / 3703 us.  Unstructured 100,000 rows, blocks of 16,
 // 69 colors: 10.3 -> 2.7 ms.
 template <int BS, int G>
@@ -816,12 +817,13 @@ __global__ __launch_bounds__((kIluThreads<BS, G>)) void k_ilu0_group(
             else hi = mid - 1;
         }
     };
-    // a pivot row: its column, place and first G upper entries, requested one pivot ahead
+    // a pivot row: its column and place, requested two pivots ahead, and its diagonal and
+    // first G upper entries, requested one ahead
     struct Pivot {
         int col, dp, p, pe, c;
         T d, v;
     };
-    auto request = [&](int i) {
+    auto place = [&](int i) {
         Pivot x;
         x.col = act && i < z ? lc[i] : 0x7fffffff;
         x.dp = -1;
@@ -830,19 +832,25 @@ __global__ __launch_bounds__((kIluThreads<BS, G>)) void k_ilu0_group(
         x.v = T(0);
         if (x.col < base) {
             x.dp = dpos[x.col];
-            x.p = (x.dp >= 0 ? x.dp + 1 : rptr[x.col]) + g;
+            x.p = rptr[x.col];
             x.pe = rptr[x.col + 1];
-            if (x.dp >= 0) x.d = val[x.dp];
-            if (x.p < x.pe) {
-                x.c = cind[x.p];
-                x.v = val[x.p];
-            }
         }
         return x;
     };
-    Pivot x = request(k);
+    auto request = [&](Pivot &x) {
+        if (x.col >= base) return;
+        x.p = (x.dp >= 0 ? x.dp + 1 : x.p) + g;
+        if (x.dp >= 0) x.d = val[x.dp];
+        if (x.p < x.pe) {
+            x.c = cind[x.p];
+            x.v = val[x.p];
+        }
+    };
+    Pivot x = place(k), nx = place(k + 1);
+    request(x);
     while (__ballot(x.col < base)) {
-        const Pivot nx = request(k + 1);
+        request(nx);
+        const Pivot h = place(k + 2);
         const bool on = x.col < base;
         T piv = T(0);
         if (on) {
@@ -861,6 +869,7 @@ __global__ __launch_bounds__((kIluThreads<BS, G>)) void k_ilu0_group(
         }
         wave_lds_sync();
         x = nx;
+        nx = h;
     }
     if constexpr (BS > 1) {
         auto sync = [&]() {  // the lanes of one block
