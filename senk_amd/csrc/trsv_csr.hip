@@ -42,9 +42,10 @@ constexpr int kCsrSpinLimit = 1 << 20, kCsrSpinCheck = 1 << 12;
 // it polls one row only, the last one still missing of its first waiting lane (the latest
 // color); when that one is there it reads all the missing ones again.  (Polling all of them,
 // up to 64 x CH lines a poll from every resident wave, slows down the rows waited for:
-// GMRES(30) of a 64^3 system 39.7 against 36.6 ms.)  Polls take the XCD's own L2 and the
-// device-coherent level in turn: the first may see a row of the same XCD sooner, the second
-// sees those of the others.
+// GMRES(30) of a 64^3 system 39.7 against 36.6 ms.)  Every other poll
+// is a plain load, which the CU's own cache may answer with the sentinel, so it only thins out
+// the polls at the device-coherent level: without it GMRES(30) of the 64^3 system takes 26.0
+// instead of 25.6 ms, the block solve of 45^3 elasticity 153 instead of 157 us.
 template <typename T, int CH>
 __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], const bool (&on)[CH],
                                            typename Bits<T>::U (&yb)[CH], unsigned *err) {
@@ -260,7 +261,9 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, co
 // consecutive rows wait for are then close together, and a poll touches a few lines instead
 // of one per entry (published by row, every resident wave's polls kept the memory system
 // busy: 61x64x67 7-point grid, 190 levels, L + U in FP64 1352 us, 581 by place; one launch
-// per level 1746).  What is left is one publish-and-poll round trip per level, about 1.5 us.
+// per level 1748).  Every poll is at the device-coherent level: a plain load may be answered
+// with the sentinel by the CU's own cache (every other poll plain 581 us, none 551; 27-point
+// 38^3 1332 and 1249).  What is left is one publish-and-poll round trip per level, about 1.45 us.
 template <typename T, bool UPPER, int CH>
 __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restrict__ seq,
                                                  const int *__restrict__ pos,
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
 #pragma unroll
         for (int q = 0; q < CH; q++)
             if (act && on[q] && yb[q] == Bits<T>::kSentinel)
-                yb[q] = (spin & 1) ? load_agent(z + cc[q]) : load_local(z + cc[q]);
+                yb[q] = load_agent(z + cc[q]);
     }
 }
 
@@ -360,10 +363,11 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
 // earlier ones like any other row).  Per row, in the order of the sequential solve
 // (senk_sparse.hpp:399-415, 436-464): first the entries of BNL x BNW blocks outside the
 // part, in rounds of about 8 gathers, then the in-part columns step by step, each finished row
-// broadcast in the wave; the next in-part block's values are held in a short register queue.
-// Bound by the levels' chain (publish, poll, in-part steps).  Elasticity 45^3, blocks of 48, 11
-// colors, L + U in FP64: FIGURE us; one lane per schedule block walking its rows, one launch per
-// color (518 lanes in flight), 3196 us.
+// broadcast in the wave; the lane's next in-part blocks wait in LDS, requested before the
+// first wait, one block read ahead of its step (in registers instead of LDS the queue spills:
+// 181-604 us).  Bound by the levels' chain (publish, poll, in-part steps).  Elasticity 45^3,
+// blocks of 48, 11 colors, L + U in FP64: 155 us; one lane per schedule block walking its rows,
+// one launch per color (518 lanes in flight), 3187 us.
 template <typename T, int BNL, int BNW, bool UPPER>
 __global__ __launch_bounds__(64 * kCsrWaves) void k_bcsr_sweep(
     SweepLevels lv, const int *__restrict__ blk_list, int bsize, int part, int bpw, const int *__restrict__ brptr,
@@ -627,8 +631,9 @@ static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
 
 // Average rows per level below which a plan's rows go through one stream, i.e. one XCD: a
 // thin level has no use for the others' bandwidth, and its waits stay on one die.  L + U in
-// FP64, one / eight streams: 7-point 12^3 (50 rows a level) 75 / 102 us, 24^3 (197) 165 /
-// 203, 40^3 (542) 315 / 350, 61x64x67 (1377) 637 / 581; 27-point 38^3 (209) 1341 / 1437.
+// FP64, one / eight streams: 7-point 12^3 (51 rows a level) 73 / 96 us, 24^3 (197) 160 /
+// 194, 40^3 (542) 309 / 334, 48^3 (776) 404 / 405, 61x64x67 (1377) 663 / 551; 27-point 38^3
+// (209) 1263 / 1352.
 constexpr double kPlanOneStream = 800;
 void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, int *streams, int *waves,
                     std::vector<int> &out) {
