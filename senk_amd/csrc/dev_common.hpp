@@ -77,6 +77,9 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 // does not depend on scheduling.
 constexpr int kPartLd = kRedMaxBlocks;  // stride between the K partial arrays of a slot
 
+// The barrier at the end of both forms keeps the other waves from the next call's writes to
+// `sh`, which every call of one instantiation shares, until the first wave has read it.
+
 template <int K>
 __device__ __forceinline__ void store_partials(const double (&v)[K], double *partials) {
     __shared__ double sh[K][kWavesPerBlock];
@@ -93,6 +96,7 @@ __device__ __forceinline__ void store_partials(const double (&v)[K], double *par
         for (int i = 0; i < kWavesPerBlock; i++) s += sh[threadIdx.x][i];
         partials[(size_t)threadIdx.x * kPartLd + blockIdx.x] = s;
     }
+    __syncthreads();
 }
 // Runtime count K <= KMAX.
 template <int KMAX>
@@ -113,6 +117,7 @@ __device__ __forceinline__ void store_partials_n(const double *v, int K, double 
         for (int i = 0; i < kWavesPerBlock; i++) s += sh[threadIdx.x][i];
         partials[(size_t)threadIdx.x * kPartLd + blockIdx.x] = s;
     }
+    __syncthreads();
 }
 // Sum of p[0..B) in a fixed order; every thread of the workgroup gets the total.  All
 // threads must call it.

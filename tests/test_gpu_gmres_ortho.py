@@ -61,3 +61,22 @@ def test_solution_of_one_cycle_matches_the_oracle(ctx, m):
     S.call("senk_gmresm_f64", ctx.h, dv.p, dc.p, dr.p, db.p, dx.p, C.c_double(nrm_b), 1, m, N, C.c_double(eps), 0,
            C.byref(res), O.P(hd), len(hd))
     assert np.linalg.norm(dx.download() - xo) <= 1e-9 * np.linalg.norm(xo)
+
+
+# the dots pass reduces two sets of products one after the other through one LDS buffer; all
+# reductions run in a fixed order, so repeated solves give the same bits
+@pytest.mark.parametrize("m", [8, 30, 50])
+def test_repeated_solves_give_the_same_bits(ctx, m):
+    rptr, cind, val = S.gen_convdiff27(33, 10.0)
+    N = len(rptr) - 1
+    b = S.gen_uniform(7, N)
+    nrm_b = float(np.linalg.norm(b))
+    d = [ctx.array(t) for t in (val, cind, rptr, b)]
+    first = None
+    for _ in range(30):
+        dx, hd, res = ctx.zeros(N), np.zeros(m), S.senk_result()
+        S.call("senk_gmresm_f64", ctx.h, *(t.p for t in d), dx.p, C.c_double(nrm_b), 1, m, N, C.c_double(1e-30), 0,
+               C.byref(res), O.P(hd), len(hd))
+        got = (hd, dx.download())
+        first = first or got
+        assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1])
