@@ -344,7 +344,7 @@ int senk_ctx_destroy(senk_ctx ctx) {
     if (c.dring_h) (void)hipHostFree(c.dring_h);
     (void)hipFree(c.red_partials);
     (void)hipFree(c.dscalars);
-    for (SweepVec &v : c.sweep)
+    for (SweepVec &v : c.sweep.v)
         if (v.p) (void)hipFree(v.p);
     (void)hipHostFree(c.sweep_err);
     (void)hipHostFree(c.hpinned);

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "senk_amd.h"
+#include "sweep_vec.hpp"
 
 namespace senk_amd {
 
@@ -45,15 +46,6 @@ constexpr int kRedMaxBlocks = 1024;  // workgroups of a reducing pass
 constexpr int kRedMaxK = 40;          // simultaneous dot products per pass
 constexpr int kRedSlots = 8;          // independent partial buffers
 
-// One of the two vectors through which the single-launch solves on caller arrays publish
-// their rows (trsv_csr.hip): `clean` leading elements of `width` bytes held the sentinel
-// before its last use as the output, which wrote the first `dirty` of them (0: reset since).
-struct SweepVec {
-    void *p = nullptr;
-    size_t bytes = 0, clean = 0, dirty = 0;
-    int width = 0;
-};
-
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -72,10 +64,8 @@ struct Ctx {
     // bytes of each
     int *dring_h = nullptr, *dring_d = nullptr;
     // single-launch solves on caller arrays: the two vectors (grown on demand, freed with the
-    // context), the one the next solve publishes in, and the time-out word in coherent
-    // pinned memory (host and device address)
-    SweepVec sweep[2];
-    int sweep_cur = 0;
+    // context), and the time-out word in coherent pinned memory (host and device address)
+    SweepVecs sweep;
     unsigned *sweep_err = nullptr, *sweep_err_d = nullptr;
     unsigned dseq = 0;  // last sequence number handed out for the ring (runs on across solves)
 };

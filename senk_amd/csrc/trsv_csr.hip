@@ -574,10 +574,11 @@ __global__ __launch_bounds__(kBlock) void k_fill_sentinel2(size_t n, T *p) {
 // ------------------------------------------------------------------ host side
 // The sweep vectors of the next solve of n rows: *z all-sentinel (filled here where the
 // last solves left less than that), *reset the vector the launch must fill in its first n
-// rows.  false: no memory (the caller takes its launch-per-level path).
+// rows; sweep_launched follows the launch.  false: no memory (the caller takes its
+// launch-per-level path).
 template <typename T>
 static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
-    SweepVec *v = c->sweep;
+    SweepVec *v = c->sweep.v;
     *ok = false;
     const size_t bytes = n * sizeof(T);
     if (!c->sweep_err || bytes >= (size_t)1 << 32) return SENK_OK;  // z is addressed by 32-bit offsets
@@ -607,25 +608,28 @@ static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
         if (st) return st;
         if (!got) return SENK_OK;
     }
-    SweepVec &u = v[c->sweep_cur], &o = v[c->sweep_cur ^ 1];
-    if (u.width != (int)sizeof(T) || u.clean < n) {
+    SweepVec &u = c->sweep.out();
+    if (c->sweep.needs_fill(n, (int)sizeof(T))) {
         k_fill_sentinel2<T><<<(int)std::min<size_t>((n + kBlock - 1) / kBlock, 2048), kBlock, 0, c->stream>>>(
             n, (T *)u.p);
         SENK_LAUNCH_CHECK();
-        u.width = (int)sizeof(T);
-        u.clean = n;
+        c->sweep.filled(n, (int)sizeof(T));
     }
-    // what this launch leaves: u written in its first n rows, o clean in them (and beyond,
-    // where o's last solve was no longer)
-    u.dirty = n;
-    if (o.width == (int)sizeof(T) && n >= o.dirty) o.clean = std::max(o.clean, n);
-    else o.clean = n;
-    o.width = (int)sizeof(T);
-    o.dirty = 0;
     *z = (T *)u.p;
-    *reset = (T *)o.p;
-    c->sweep_cur ^= 1;
+    *reset = (T *)c->sweep.next().p;
     *ok = true;
+    return SENK_OK;
+}
+// The status of the launch that took the vectors of sweep_vectors<T>(n).
+template <typename T>
+static int sweep_launched(Ctx *c, size_t n) {
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) {
+        c->sweep.solved(n, (int)sizeof(T));
+        return SENK_OK;
+    }
+    c->sweep.spoiled();
+    SENK_HIP(e);
     return SENK_OK;
 }
 
@@ -701,8 +705,9 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
     T *z = nullptr, *reset = nullptr;
     if (s.dblk) {
         if (BS != 1 || !s.dseq || !s.dpos || s.seq_upper != upper) return SENK_OK;
+        const size_t nz = (size_t)s.seq_waves * s.streams * 64;
         bool ok = false;
-        SENK_TRY(sweep_vectors<T>(c, (size_t)s.seq_waves * s.streams * 64, &z, &reset, &ok));
+        SENK_TRY(sweep_vectors<T>(c, nz, &z, &reset, &ok));
         if (!ok) return SENK_OK;
         const int grid = kXcds * s.seq_waves;
         // rounds of 4 where no row has more entries, else of 16: a second round costs its own
@@ -715,7 +720,7 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
         else if (s.max_ext <= 4) SENK_CSR_ROWS(false, 4);
         else SENK_CSR_ROWS(false, 16);
 #undef SENK_CSR_ROWS
-        SENK_LAUNCH_CHECK();
+        SENK_TRY(sweep_launched<T>(c, nz));
         *done = true;
         return SENK_OK;
     }
@@ -744,10 +749,10 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
         SENK_CSR_SWEEP(16)
         SENK_CSR_SWEEP(32)
         SENK_CSR_SWEEP(64)
-        default: return SENK_ERR_UNSUPPORTED;
+        default: return SENK_ERR_UNSUPPORTED;  // not reached: BS divides 64
     }
 #undef SENK_CSR_SWEEP
-    SENK_LAUNCH_CHECK();
+    SENK_TRY(sweep_launched<T>(c, (size_t)N));
     *done = true;
     return SENK_OK;
 }
@@ -779,12 +784,9 @@ int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int
     SweepLevels lv;
     int tickets = 0;
     if (!sweep_levels(s, upper, 1, bpw, &lv, &tickets)) return SENK_OK;
-    T *z = nullptr, *reset = nullptr;
-    bool ok = false;
-    SENK_TRY(sweep_vectors<T>(c, (size_t)N, &z, &reset, &ok));
-    if (!ok) return SENK_OK;
+    decltype(&bcsr_sweep<T, 1, 1>) launch = nullptr;
 #define SENK_BCSR_SWEEP(A, B) \
-    case 16 * A + B: bcsr_sweep<T, A, B>(c, lv, tickets, s, upper, part, bpw, brptr, bcind, bval, x, y, z, reset); break
+    case 16 * A + B: launch = bcsr_sweep<T, A, B>; break
     switch (16 * bnl + bnw) {
         SENK_BCSR_SWEEP(1, 1);
         SENK_BCSR_SWEEP(2, 1);
@@ -801,7 +803,12 @@ int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int
         default: return SENK_ERR_UNSUPPORTED;  // as the launch per level
     }
 #undef SENK_BCSR_SWEEP
-    SENK_LAUNCH_CHECK();
+    T *z = nullptr, *reset = nullptr;
+    bool ok = false;
+    SENK_TRY(sweep_vectors<T>(c, (size_t)N, &z, &reset, &ok));
+    if (!ok) return SENK_OK;
+    launch(c, lv, tickets, s, upper, part, bpw, brptr, bcind, bval, x, y, z, reset);
+    SENK_TRY(sweep_launched<T>(c, (size_t)N));
     *done = true;
     return SENK_OK;
 }

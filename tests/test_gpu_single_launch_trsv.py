@@ -193,3 +193,29 @@ def test_bcsr_blocks_in_any_order(ctx, bnl, bnw, bsize):
     so a few tens of roundings each)."""
     t, u, yl, yu = _bcsr(ctx, 8, bnl, bnw, bsize, shuffle=True)
     assert relerr(t, yl) <= 1e-13 and relerr(u, yu) <= 1e-13
+
+
+def _refused(ctx, bnl, bnw, n):
+    """A block solve of n rows in a shape that no kernel takes: SENK_ERR_UNSUPPORTED (9)."""
+    rptr = np.zeros(n // bnl + 1, np.int32)
+    d = [ctx.array(t) for t in (np.zeros(1), np.zeros(1, np.int32), rptr, np.ones(n))]
+    dy = ctx.zeros(n)
+    cptr = np.array([0, 1], np.int32)
+    assert S.lib().senk_sptrsv_bcsr_l_abmc_f64(ctx.h, *(t.p for t in d), dy.p, n, O.P(cptr), 1, n, bnl, bnw) == 9
+    assert S.lib().senk_sptrsv_bcsr_u_abmc_f64(ctx.h, *(t.p for t in d), dy.p, n, O.P(cptr), 1, n, bnl, bnw) == 9
+
+
+@pytest.mark.parametrize("bnl,bnw", [(5, 5), (6, 3), (6, 6), (16, 16)])
+def test_a_refused_block_shape_leaves_the_next_solves_right(ctx, bnl, bnw):
+    """The refusal neither uses nor turns over the vectors the solves share: before any other
+    solve of a context, and between two solves of one size with different right-hand sides."""
+    mats = [S.gen_vardiff7(8, s, 4.0, 1.5) for s in (3, 4)]
+    with S.Context(0) as fresh:
+        _refused(fresh, bnl, bnw, 240)
+        _abmc_case(fresh, mats[0], 8, "connect", np.float64)
+    for k in range(3):  # an odd and an even number of refusals between solves
+        _abmc_case(ctx, mats[k & 1], 8, "connect", np.float64)
+        for _ in range(k + 1):
+            _refused(ctx, bnl, bnw, 480)
+        _abmc_case(ctx, mats[(k + 1) & 1], 8, "connect", np.float64)
+        _plan_case(ctx, mats[k & 1], np.float64)
