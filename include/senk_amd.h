@@ -58,6 +58,10 @@ typedef struct senk_ctx_s *senk_ctx;
 int senk_ctx_create(int device, senk_ctx *out);
 int senk_ctx_destroy(senk_ctx ctx);
 int senk_ctx_synchronize(senk_ctx ctx);
+/* No reference counterpart: how often a wait of the single-launch triangular solves on caller
+ * arrays polls (at least half a microsecond each) before it gives up and the solve's result
+ * becomes invalid (SENK_ERR_TIMEOUT).  0 restores the default, 2^22. */
+int senk_ctx_set_trsv_polls(senk_ctx ctx, int polls);
 int senk_device_count(int *count);
 int senk_device_malloc(senk_ctx ctx, size_t bytes, void **dptr);
 int senk_device_free(senk_ctx ctx, void *dptr);

@@ -358,6 +358,12 @@ int senk_ctx_synchronize(senk_ctx ctx) {
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
     return ctx_sweep_check(&ctx->c);
 }
+int senk_ctx_set_trsv_polls(senk_ctx ctx, int polls) {
+    CTX_CHECK(ctx);
+    if (polls < 0) return SENK_ERR_ARG;
+    ctx->c.sweep_polls = polls ? std::min(polls, 1 << 29) : senk_amd::kSweepPolls;
+    return SENK_OK;
+}
 int senk_device_malloc(senk_ctx ctx, size_t bytes, void **dptr) {
     CTX_CHECK(ctx);
     if (!dptr) return SENK_ERR_ARG;

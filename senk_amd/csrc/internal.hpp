@@ -46,6 +46,11 @@ constexpr int kRedMaxBlocks = 1024;  // workgroups of a reducing pass
 constexpr int kRedMaxK = 40;          // simultaneous dot products per pass
 constexpr int kRedSlots = 8;          // independent partial buffers
 
+// Polls at the device-coherent level after which a wait of the single-launch solves on caller
+// arrays gives up.  Each is a round trip past the caches (half a microsecond or more), so an
+// ordinary wait of up to two seconds is never given up.
+constexpr int kSweepPolls = 1 << 22;
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -66,6 +71,7 @@ struct Ctx {
     // single-launch solves on caller arrays: the two vectors (grown on demand, freed with the
     // context), and the time-out word in coherent pinned memory (host and device address)
     SweepVecs sweep;
+    int sweep_polls = kSweepPolls;
     unsigned *sweep_err = nullptr, *sweep_err_d = nullptr;
     unsigned dseq = 0;  // last sequence number handed out for the ring (runs on across solves)
 };

@@ -31,12 +31,17 @@ struct SweepLevels {
     int n;
     int ticket[kSweepMaxLevels], unit0[kSweepMaxLevels], units[kSweepMaxLevels];
 };
+// What a launch's waits need: the context's time-out word and the polls after which a wait
+// gives up.
+struct SweepWait {
+    unsigned *err;
+    int limit;
+};
 
 namespace {
 constexpr int kCsrWaves = 4;  // waves per workgroup, each with rows (and staged entries) of its own
-// Polls before a wait gives up (a second or more), and how often it looks whether another
-// wait has already given up.
-constexpr int kCsrSpinLimit = 1 << 20, kCsrSpinCheck = 1 << 12;
+// How often (in polls, a power of two) a wait looks whether another wait has already given up.
+constexpr int kCsrSpinCheck = 1 << 12;
 
 // Waits until every row cc[q] (on[q]) is published in z, its bits in yb.  While a wave waits
 // it polls one row only, the last one still missing of its first waiting lane (the latest
@@ -45,10 +50,11 @@ constexpr int kCsrSpinLimit = 1 << 20, kCsrSpinCheck = 1 << 12;
 // GMRES(30) of a 64^3 system 39.7 against 36.6 ms.)  Every other poll
 // is a plain load, which the CU's own cache may answer with the sentinel, so it only thins out
 // the polls at the device-coherent level: without it GMRES(30) of the 64^3 system takes 26.0
-// instead of 25.6 ms, the block solve of 45^3 elasticity 153 instead of 157 us.
+// instead of 25.6 ms, the block solve of 45^3 elasticity 153 instead of 157 us.  The limit is
+// on the device-coherent ones, so that many round trips bound the wait from below.
 template <typename T, int CH>
 __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], const bool (&on)[CH],
-                                           typename Bits<T>::U (&yb)[CH], unsigned *err) {
+                                           typename Bits<T>::U (&yb)[CH], SweepWait wt) {
     int want = -1;  // the last missing row of this lane
 #pragma unroll
     for (int q = 0; q < CH; q++)
@@ -58,10 +64,10 @@ __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], cons
         const T *p = z + __builtin_amdgcn_readlane(want, __ffsll((long long)b) - 1);
         while ((spin & 1 ? load_local(p) : load_agent(p)) == Bits<T>::kSentinel) {
             spin++;
-            if (spin >= kCsrSpinLimit ||
+            if ((spin >> 1) >= wt.limit ||
                 ((spin & (kCsrSpinCheck - 1)) == 0 &&
-                 __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
-                __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                 __hip_atomic_load(wt.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+                __hip_atomic_store(wt.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return;
             }
             __builtin_amdgcn_s_sleep(1);
@@ -105,7 +111,7 @@ template <typename T>
 constexpr int kCsrCap = 10 * 1024 / (int)(sizeof(T) + sizeof(int));
 
 template <typename T, int BS, bool UPPER, typename FC, typename FV>
-__device__ __forceinline__ T solve_row(T t, int s, int e, bool active, int base, const T *z, unsigned *err, FC C,
+__device__ __forceinline__ T solve_row(T t, int s, int e, bool active, int base, const T *z, SweepWait wt, FC C,
                                        FV V) {
     using U = typename Bits<T>::U;
     constexpr int CH = 8;
@@ -134,7 +140,7 @@ __device__ __forceinline__ T solve_row(T t, int s, int e, bool active, int base,
 #pragma unroll
         for (int q = 0; q < CH; q++)
             if (on[q]) yb[q] = load_local(ixp<true>(z, cc[q]));
-        await_rows<T, CH>(z, cc, on, yb, err);
+        await_rows<T, CH>(z, cc, on, yb, wt);
 #pragma unroll
         for (int q = 0; q < CH; q++)
             if (on[q]) t -= vv[q] * __builtin_bit_cast(T, yb[q]);
@@ -198,7 +204,7 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, co
                                                               const int *__restrict__ cind,
                                                               const T *__restrict__ val, const T *x, T *y, T *z,
                                                               T *reset, const double *__restrict__ in_scale,
-                                                              unsigned *err, const int *__restrict__ stop) {
+                                                              SweepWait wt, const int *__restrict__ stop) {
     __shared__ T sv[kCsrWaves][kCsrCap<T>];
     __shared__ int sc[kCsrWaves][kCsrCap<T>];
     const int xs = (int)(blockIdx.x % kXcds), j = (int)(blockIdx.x / kXcds);
@@ -240,10 +246,10 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, co
                 }
         }
         wave_lds_sync();
-        t = solve_row<T, BS, UPPER>(t, s - e0, e - e0, active, base, z, err, [&](int i) { return sc[wv][i]; },
+        t = solve_row<T, BS, UPPER>(t, s - e0, e - e0, active, base, z, wt, [&](int i) { return sc[wv][i]; },
                                     [&](int i) { return sv[wv][i]; });
     } else {
-        t = solve_row<T, BS, UPPER>(t, s, e, active, base, z, err, [&](int i) { return cind[i]; },
+        t = solve_row<T, BS, UPPER>(t, s, e, active, base, z, wt, [&](int i) { return cind[i]; },
                                     [&](int i) { return val[i]; });
     }
     if (active) {
@@ -269,7 +275,7 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
                                                  const int *__restrict__ pos,
                                                  const int *__restrict__ rptr, const int *__restrict__ cind,
                                                  const T *__restrict__ val, const T *x, T *y, T *z, T *reset,
-                                                 const double *__restrict__ in_scale, unsigned *err,
+                                                 const double *__restrict__ in_scale, SweepWait wt,
                                                  const int *__restrict__ stop) {
     using U = typename Bits<T>::U;
     const int xs = (int)(blockIdx.x % kXcds), w = (int)(blockIdx.x / kXcds);
@@ -337,12 +343,12 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
             }
             continue;
         }
-        if (spin >= kCsrSpinLimit ||
+        if (spin >= wt.limit ||
             ((spin & (kCsrSpinCheck - 1)) == kCsrSpinCheck - 1 &&
-             __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+             __hip_atomic_load(wt.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
             // give up: publish a NaN so that the rows behind this one end too
             if (act) {
-                __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(wt.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 t = __builtin_nan("");
                 store_agent(z + mine, canonical(t));
                 y[row] = t;
@@ -371,7 +377,7 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
 template <typename T, int BNL, int BNW, bool UPPER>
 __global__ __launch_bounds__(64 * kCsrWaves) void k_bcsr_sweep(
     SweepLevels lv, const int *__restrict__ blk_list, int bsize, int part, int bpw, const int *__restrict__ brptr,
-    const int *__restrict__ bcind, const T *__restrict__ bval, const T *x, T *y, T *z, T *reset, unsigned *err) {
+    const int *__restrict__ bcind, const T *__restrict__ bval, const T *x, T *y, T *z, T *reset, SweepWait wt) {
     using U = typename Bits<T>::U;
     constexpr int BS = BNL * BNW, BREM = BNL / BNW;
     constexpr int CB = BNW >= 8 ? 1 : (8 + BNW - 1) / BNW;  // blocks per round
@@ -479,7 +485,7 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_bcsr_sweep(
 #pragma unroll
             for (int q = 0; q < CB * BNW; q++)
                 if (on[q]) yb[q] = load_local(ixp<true>(z, cc[q]));
-            await_rows<T, CB * BNW>(z, cc, on, yb, err);
+            await_rows<T, CB * BNW>(z, cc, on, yb, wt);
 #pragma unroll
             for (int q = 0; q < CB * BNW; q++)
                 if (on[q]) t -= vv[q] * __builtin_bit_cast(T, yb[q]);
@@ -714,7 +720,7 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
         // chain of dependent loads after the last row of the first is there
 #define SENK_CSR_ROWS(UP, CH)                                                                                      \
     k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.streams, s.dseq, s.dpos, rptr, cind, val, x, y, z, reset, \
-                                                      UP ? nullptr : in_scale, c->sweep_err_d, stop)
+                                                      UP ? nullptr : in_scale, SweepWait{c->sweep_err_d, c->sweep_polls}, stop)
         if (upper && s.max_ext <= 4) SENK_CSR_ROWS(true, 4);
         else if (upper) SENK_CSR_ROWS(true, 16);
         else if (s.max_ext <= 4) SENK_CSR_ROWS(false, 4);
@@ -735,10 +741,10 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
     case B:                                                                                                      \
         if (upper)                                                                                               \
             k_csr_sweep<T, B, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z, reset, \
-                                                                            nullptr, c->sweep_err_d, stop);      \
+                                                                            nullptr, SweepWait{c->sweep_err_d, c->sweep_polls}, stop);      \
         else                                                                                                     \
             k_csr_sweep<T, B, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z,       \
-                                                                             reset, in_scale, c->sweep_err_d,    \
+                                                                             reset, in_scale, SweepWait{c->sweep_err_d, c->sweep_polls},    \
                                                                              stop);                              \
         break;
     switch (BS) {
@@ -767,10 +773,10 @@ static void bcsr_sweep(Ctx *c, const SweepLevels &lv, int tickets, const Schedul
     const int grid = kXcds * tickets;
     if (upper)
         k_bcsr_sweep<T, BNL, BNW, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
-            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, c->sweep_err_d);
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, SweepWait{c->sweep_err_d, c->sweep_polls});
     else
         k_bcsr_sweep<T, BNL, BNW, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
-            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, c->sweep_err_d);
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, SweepWait{c->sweep_err_d, c->sweep_polls});
 }
 template <typename T>
 int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,

@@ -219,3 +219,43 @@ def test_a_refused_block_shape_leaves_the_next_solves_right(ctx, bnl, bnw):
             _refused(ctx, bnl, bnw, 480)
         _abmc_case(ctx, mats[(k + 1) & 1], 8, "connect", np.float64)
         _plan_case(ctx, mats[k & 1], np.float64)
+
+
+def _gives_up(ctx, solve):
+    """`solve` under a limit of one poll: its waits give up, and the context says so once."""
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 1) == 0
+    try:
+        solve()
+        return S.lib().senk_ctx_synchronize(ctx.h)
+    finally:
+        assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 0) == 0
+
+
+def _chain(ctx, n, dt=np.float64):
+    """The L solve of a tridiagonal system on a plan (every row waits on the one before): a
+    function that runs it, and its result's array and expected values."""
+    rptr, cind, val = _tridiagonal(n)
+    L, _ = (_typed(f, dt) for f in ilu_factors(dict(val=val, cind=cind, rptr=rptr)))
+    x = np.random.default_rng(n).uniform(-1, 1, n).astype(dt)
+    y = np.zeros_like(x)
+    getattr(O.orc(), "or_sptrsv_l_" + ("d" if dt == np.float64 else "f"))(*(O.P(t) for t in L), O.P(x), O.P(y), n)
+    plan = C.c_void_p()
+    S.call("senk_trsv_plan_create", ctx.h, O.P(L[2]), O.P(L[1]), n, 0, C.byref(plan))
+    d = [ctx.array(t) for t in (*L, x)]
+    dy = ctx.zeros(n, dt)
+    s = "f64" if dt == np.float64 else "f32"
+
+    def run():
+        S.call("senk_sptrsv_csr_l_" + s, ctx.h, plan, *(t.p for t in d), dy.p, n)
+
+    return run, dy, y
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_poll_limit(ctx, dt):
+    run, dy, y = _chain(ctx, 500, dt)
+    assert _gives_up(ctx, run) == 11
+    assert S.lib().senk_ctx_synchronize(ctx.h) == 0
+    run()
+    assert np.array_equal(dy.download(), y)
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, -1) == 1
