@@ -42,8 +42,10 @@ enum senk_status {
     SENK_ERR_SCHEDULE = 10,      /* a factor entry couples two blocks scheduled together       */
     SENK_ERR_TIMEOUT = 11,       /* a single-launch triangular solve gave up waiting on an
                                     earlier level (the result of that solve is invalid);
-                                    solves on caller arrays report it at the next driver end,
-                                    senk_ctx_synchronize or senk_memcpy_dtoh                 */
+                                    solves on caller arrays report it at the next call that
+                                    waits for the context to hand results to the host: a
+                                    driver or senk_solve, senk_dot / senk_nrm2,
+                                    senk_memcpy_dtoh, senk_ctx_synchronize, senk_prec_check  */
     SENK_ERR_IO = 12,            /* a file could not be opened or read                         */
     SENK_ERR_FORMAT = 13         /* a file is not a MatrixMarket matrix the reader supports    */
 };

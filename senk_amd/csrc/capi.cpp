@@ -674,10 +674,11 @@ static int bcsr_seq(senk_ctx ctx, const T *dbval, const int *dbcind, const int *
     if (N % bnl || bnl % bnw) return SENK_ERR_DIVISIBILITY;
     Schedule s;
     SENK_TRY(bcsr_seq_schedule(ctx, dbcind, dbrptr, N, bnl, bnw, upper, &s));
-    const int st = launch_sptrsv_bcsr<T>(&ctx->c, s, upper, N, bnl, bnw, dbrptr, dbcind, dbval, dx, dy);
+    int st = launch_sptrsv_bcsr<T>(&ctx->c, s, upper, N, bnl, bnw, dbrptr, dbcind, dbval, dx, dy);
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
     (void)hipFree(s.dblk);
-    return st;
+    const int late = ctx_sweep_check(&ctx->c);
+    return st ? st : late;
 }
 extern "C" {
 int senk_sptrsv_bcsr_l_abmc_f64(senk_ctx ctx, const double *dbval, const int *dbcind, const int *dbrptr,
@@ -754,7 +755,7 @@ int senk_dot_f64(senk_ctx ctx, const double *dx, const double *dy, int N, double
     SENK_HIP(hipMemcpyAsync(ctx->c.hpinned, ctx->c.dscalars, sizeof(double), hipMemcpyDeviceToHost, ctx->c.stream));
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
     *result = ctx->c.hpinned[0];
-    return SENK_OK;
+    return ctx_sweep_check(&ctx->c);
 }
 int senk_nrm2_f64_dev(senk_ctx ctx, const double *dx, int N, double *dres) { return senk_dot_f64_dev(ctx, dx, dx, N, dres); }
 int senk_nrm2_f64(senk_ctx ctx, const double *dx, int N, double *result) {
@@ -809,7 +810,7 @@ int senk_dot_f32(senk_ctx ctx, const float *dx, const float *dy, int N, double *
     SENK_HIP(hipMemcpyAsync(ctx->c.hpinned, ctx->c.dscalars, sizeof(double), hipMemcpyDeviceToHost, ctx->c.stream));
     SENK_HIP(hipStreamSynchronize(ctx->c.stream));
     *result = ctx->c.hpinned[0];
-    return SENK_OK;
+    return ctx_sweep_check(&ctx->c);
 }
 int senk_nrm2_f32(senk_ctx ctx, const float *dx, int N, double *result) {
     SENK_TRY(senk_dot_f32(ctx, dx, dx, N, result));
@@ -924,7 +925,12 @@ static int run_twin(senk_ctx ctx, const MatView &A, const PrecView &M, SolvePara
                     senk_result *res, double *hist, int hist_cap) {
     senk_result tmp;
     if (!res) res = &tmp;
-    SENK_TRY(krylov_solve<double>(&ctx->c, A, M, db, dx, p, res, hist, hist_cap));
+    const int st = krylov_solve<double>(&ctx->c, A, M, db, dx, p, res, hist, hist_cap);
+    if (st) {  // no give-up of it is left for a later call to report
+        (void)hipStreamSynchronize(ctx->c.stream);
+        (void)ctx_sweep_check(&ctx->c);
+        return st;
+    }
     return finish(ctx, A, db, dx, p.nrm_b, res);
 }
 
@@ -1684,7 +1690,10 @@ int senk_prec_check(senk_prec M) {
     if (!M) return SENK_ERR_ARG;
     const int a = senk_amd::tri_layout_check(&M->ctx->c, &M->lt);
     const int b = senk_amd::tri_layout_check(&M->ctx->c, &M->ut);
-    return a ? a : b;
+    // factors without the sliced layout solve as caller arrays do
+    SENK_HIP(hipStreamSynchronize(M->ctx->c.stream));
+    const int s = ctx_sweep_check(&M->ctx->c);
+    return a ? a : b ? b : s;
 }
 int senk_prec_factor_nnz(senk_prec M, int *lnnz, int *unnz, int *nlev_l, int *nlev_u) {
     if (!M) return SENK_ERR_ARG;
@@ -1769,12 +1778,11 @@ int senk_solve(senk_ctx ctx, senk_mat A, senk_prec M, const double *db, double *
         pv.in32 = (float *)buf;
         pv.out32 = pv.in32 + ld;
     }
+    int st = SENK_OK;
     if (o->mixed == 1 || o->mixed == 2) {
         if (!A->v32 || (M && !M->view.l32 && !pv.f16)) return SENK_ERR_ARG;
-        if (o->mixed == 2)
-            SENK_TRY(nested_solve(&ctx->c, A->view, pv, db, dx, *o, nrm_b, res, hist, hist_cap));
-        else
-            SENK_TRY(ir_solve(&ctx->c, A->view, pv, db, dx, *o, nrm_b, res, hist, hist_cap));
+        st = o->mixed == 2 ? nested_solve(&ctx->c, A->view, pv, db, dx, *o, nrm_b, res, hist, hist_cap)
+                           : ir_solve(&ctx->c, A->view, pv, db, dx, *o, nrm_b, res, hist, hist_cap);
     } else {
         SolveParams p;
         p.solver = o->solver;
@@ -1786,7 +1794,11 @@ int senk_solve(senk_ctx ctx, senk_mat A, senk_prec M, const double *db, double *
         p.ortho = o->ortho;
         p.check_every = o->check_every;
         p.verbose = o->verbose;
-        SENK_TRY(krylov_solve<double>(&ctx->c, A->view, pv, db, dx, p, res, hist, hist_cap));
+        st = krylov_solve<double>(&ctx->c, A->view, pv, db, dx, p, res, hist, hist_cap);
+    }
+    if (st) {  // no give-up of it is left for a later call to report
+        if (M) (void)senk_prec_check(M);
+        return st;
     }
     double tr = 0;
     SENK_TRY(true_relres(&ctx->c, A->view, db, dx, nrm_b, &tr));
@@ -1834,7 +1846,9 @@ int senk_gnn_loss_grad(senk_gnn g, senk_mat A, senk_prec M, const float *dR, int
 int senk_gnn_loss_grad_pairs(senk_gnn g, senk_mat A, senk_prec M, const float *dR, const float *dZ, int nvec,
                              double *loss, double *grad) {
     if (!g || !A || !M || !dR || nvec <= 0 || (!dZ && !M->view.l32) || !A->v32) return SENK_ERR_ARG;
-    return gnn_loss_grad(g, A->view, plain_view(M), dR, dZ, nvec, loss, grad);
+    const int st = gnn_loss_grad(g, A->view, plain_view(M), dR, dZ, nvec, loss, grad);
+    const int late = senk_prec_check(M);
+    return st ? st : late;
 }
 int senk_gnn_train(senk_gnn g, int nmat, const senk_mat *A, const senk_prec *M, const float *const *dR,
                    const int *nvec, int epochs, int batch, double lr, unsigned seed, double *loss_hist, int verbose) {
@@ -1852,7 +1866,12 @@ int senk_gnn_train_pairs(senk_gnn g, int nmat, const senk_mat *A, const senk_pre
         av[k] = A[k]->view;
         pv[k] = plain_view(M[k]);
     }
-    return gnn_train(g, nmat, av.data(), pv.data(), dR, dZ, nvec, epochs, batch, lr, seed, loss_hist, verbose);
+    int st = gnn_train(g, nmat, av.data(), pv.data(), dR, dZ, nvec, epochs, batch, lr, seed, loss_hist, verbose);
+    for (int k = 0; k < nmat; k++) {
+        const int late = senk_prec_check(M[k]);
+        if (!st) st = late;
+    }
+    return st;
 }
 int senk_gnn_collect_nested(senk_ctx ctx, senk_mat A, senk_prec M, const double *db, const senk_solve_opts *opts,
                             float *dR, float *dZ, int cap, int *count) {
@@ -1874,13 +1893,16 @@ int senk_gnn_collect_nested(senk_ctx ctx, senk_mat A, senk_prec M, const double 
     (void)hipStreamSynchronize(ctx->c.stream);
     (void)hipFree(dx);
     *count = rec.count;
-    return st;
+    const int late = senk_prec_check(M);
+    return st ? st : late;
 }
 int senk_gnn_collect(senk_ctx ctx, senk_mat A, senk_prec M, const double *db, const double *dxstar, int m,
                      int ncycles, double *dR, double *dE, int *count) {
     CTX_CHECK(ctx);
     if (!A || !M || !db || !dR || m <= 0 || ncycles <= 0 || !count) return SENK_ERR_ARG;
-    return collect_pairs(&ctx->c, A->view, plain_view(M), db, dxstar, m, ncycles, dR, dE, count);
+    const int st = collect_pairs(&ctx->c, A->view, plain_view(M), db, dxstar, m, ncycles, dR, dE, count);
+    const int late = senk_prec_check(M);
+    return st ? st : late;
 }
 int senk_prec_attach_gnn(senk_prec M, senk_gnn g) {
     if (!M) return SENK_ERR_ARG;

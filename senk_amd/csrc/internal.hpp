@@ -73,13 +73,15 @@ struct Ctx {
     SweepVecs sweep;
     int sweep_polls = kSweepPolls;
     unsigned *sweep_err = nullptr, *sweep_err_d = nullptr;
+    unsigned sweep_tag = 0;  // number of the last such launch: what the word holds if it gave up
     unsigned dseq = 0;  // last sequence number handed out for the ring (runs on across solves)
 };
 // Creates the context's reusable events and pinned ring on first use.
 int ctx_events(Ctx *c);
 
 // SENK_ERR_TIMEOUT (once) if a single-launch solve on caller arrays gave up a wait; the
-// stream must be synchronised.
+// stream must be synchronised.  Every call that waits for the stream to hand results to the
+// host ends with it.
 int ctx_sweep_check(Ctx *c);
 
 int ctx_work(Ctx *c, size_t bytes, void **out);

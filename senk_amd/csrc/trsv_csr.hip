@@ -31,10 +31,11 @@ struct SweepLevels {
     int n;
     int ticket[kSweepMaxLevels], unit0[kSweepMaxLevels], units[kSweepMaxLevels];
 };
-// What a launch's waits need: the context's time-out word and the polls after which a wait
-// gives up.
+// What a launch's waits need: the context's time-out word, the launch's number, which a wait
+// that gives up writes there, and the polls after which it does.  The other waits of the
+// launch then give up as well; those of later launches, whatever the word still holds, do not.
 struct SweepWait {
-    unsigned *err;
+    unsigned *err, tag;
     int limit;
 };
 
@@ -66,8 +67,8 @@ __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], cons
             spin++;
             if ((spin >> 1) >= wt.limit ||
                 ((spin & (kCsrSpinCheck - 1)) == 0 &&
-                 __hip_atomic_load(wt.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
-                __hip_atomic_store(wt.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                 __hip_atomic_load(wt.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == wt.tag)) {
+                __hip_atomic_store(wt.err, wt.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return;
             }
             __builtin_amdgcn_s_sleep(1);
@@ -345,10 +346,10 @@ __global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restr
         }
         if (spin >= wt.limit ||
             ((spin & (kCsrSpinCheck - 1)) == kCsrSpinCheck - 1 &&
-             __hip_atomic_load(wt.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+             __hip_atomic_load(wt.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == wt.tag)) {
             // give up: publish a NaN so that the rows behind this one end too
             if (act) {
-                __hip_atomic_store(wt.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(wt.err, wt.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 t = __builtin_nan("");
                 store_agent(z + mine, canonical(t));
                 y[row] = t;
@@ -626,6 +627,10 @@ static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
     *ok = true;
     return SENK_OK;
 }
+static SweepWait sweep_wait(Ctx *c) {
+    if (++c->sweep_tag == 0) c->sweep_tag = 1;  // 0: nothing gave up
+    return SweepWait{c->sweep_err_d, c->sweep_tag, c->sweep_polls};
+}
 // The status of the launch that took the vectors of sweep_vectors<T>(n).
 template <typename T>
 static int sweep_launched(Ctx *c, size_t n) {
@@ -720,7 +725,7 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
         // chain of dependent loads after the last row of the first is there
 #define SENK_CSR_ROWS(UP, CH)                                                                                      \
     k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.streams, s.dseq, s.dpos, rptr, cind, val, x, y, z, reset, \
-                                                      UP ? nullptr : in_scale, SweepWait{c->sweep_err_d, c->sweep_polls}, stop)
+                                                      UP ? nullptr : in_scale, sweep_wait(c), stop)
         if (upper && s.max_ext <= 4) SENK_CSR_ROWS(true, 4);
         else if (upper) SENK_CSR_ROWS(true, 16);
         else if (s.max_ext <= 4) SENK_CSR_ROWS(false, 4);
@@ -741,10 +746,10 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
     case B:                                                                                                      \
         if (upper)                                                                                               \
             k_csr_sweep<T, B, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z, reset, \
-                                                                            nullptr, SweepWait{c->sweep_err_d, c->sweep_polls}, stop);      \
+                                                                            nullptr, sweep_wait(c), stop);      \
         else                                                                                                     \
             k_csr_sweep<T, B, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z,       \
-                                                                             reset, in_scale, SweepWait{c->sweep_err_d, c->sweep_polls},    \
+                                                                             reset, in_scale, sweep_wait(c),    \
                                                                              stop);                              \
         break;
     switch (BS) {
@@ -773,10 +778,10 @@ static void bcsr_sweep(Ctx *c, const SweepLevels &lv, int tickets, const Schedul
     const int grid = kXcds * tickets;
     if (upper)
         k_bcsr_sweep<T, BNL, BNW, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
-            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, SweepWait{c->sweep_err_d, c->sweep_polls});
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, sweep_wait(c));
     else
         k_bcsr_sweep<T, BNL, BNW, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
-            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, SweepWait{c->sweep_err_d, c->sweep_polls});
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, sweep_wait(c));
 }
 template <typename T>
 int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,

@@ -259,3 +259,89 @@ def test_poll_limit(ctx, dt):
     run()
     assert np.array_equal(dy.download(), y)
     assert S.lib().senk_ctx_set_trsv_polls(ctx.h, -1) == 1
+
+
+def test_a_wait_given_up_ends_only_its_own_solve(ctx):
+    """The time-out word still set by an earlier solve (nothing has read it) does not end the
+    waits of a later one, here of some 40 ms."""
+    short, _, _ = _chain(ctx, 500)
+    long, dy, y = _chain(ctx, 30000)
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 1) == 0
+    short()
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 0) == 0
+    long()
+    assert S.lib().senk_ctx_synchronize(ctx.h) == 11  # the short one's
+    assert np.array_equal(dy.download(), y)
+
+
+def _abmc():
+    rptr, cind, val = S.gen_vardiff7(20, 3, 4.0, 1.5)
+    sy = abmc_system(rptr, cind, val, 8)
+    sy["N"] = len(rptr) - 1
+    sy["x"] = np.random.default_rng(8).uniform(-1, 1, sy["N"])
+    return sy
+
+
+def test_a_wait_given_up_is_reported_by_the_next_result(ctx):
+    """Dot products and copies to the host, the sequential block form (which synchronises by
+    itself) and a driver report it, once; the same calls are right again afterwards."""
+    run, dy, y = _chain(ctx, 500)
+    n, dot = len(y), C.c_double()
+    buf = np.zeros(n)
+    for read in (lambda: S.lib().senk_dot_f64(ctx.h, dy.p, dy.p, n, C.byref(dot)),
+                 lambda: S.lib().senk_memcpy_dtoh(ctx.h, O.P(buf), dy.p, C.c_size_t(8 * n))):
+        assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 1) == 0
+        run()
+        assert read() == 11 and read() == 0
+        assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 0) == 0
+    rptr, cind, val = _tridiagonal(200)
+    L, _ = ilu_factors(dict(val=val, cind=cind, rptr=rptr))
+    bl = S.csr2bcsr(*L, 200, 2, 2)
+    d = [ctx.array(t) for t in (*bl, np.ones(200))]
+    dz = ctx.zeros(200)
+    seq = lambda: S.lib().senk_sptrsv_bcsr_l_f64(ctx.h, *(t.p for t in d), dz.p, 200, 2, 2)
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 1) == 0
+    assert seq() == 11
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 0) == 0
+    assert seq() == 0
+    sy = _abmc()
+    L, U = ilu_factors(sy)
+    d = [ctx.array(t) for t in (sy["val"], sy["cind"], sy["rptr"], *L, *U, sy["x"])]
+    dx, res = ctx.zeros(sy["N"]), S.senk_result()
+    nrm_b = float(np.linalg.norm(sy["x"]))
+    drv = lambda: S.lib().senk_abmc_ilu_gmresm_f64(ctx.h, *(t.p for t in d[:9]), O.P(sy["cptr"]), sy["nc"], 8, d[9].p,
+                                                   dx.p, C.c_double(nrm_b), 100, 30, sy["N"], C.c_double(1e-8), 0,
+                                                   C.byref(res), None, 0)
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 1) == 0
+    assert drv() == 11
+    assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 0) == 0
+    dx.zero()
+    assert drv() == 0 and res.converged == 1
+
+
+@pytest.mark.parametrize("kind", ["ilu0", "ilub"])
+def test_handles_without_the_sliced_layout_report_a_wait_given_up(ctx, kind):
+    sy = _abmc()
+    N = sy["N"]
+    A, M = C.c_void_p(), C.c_void_p()
+    S.call("senk_mat_create", ctx.h, N, O.P(sy["rptr"]), O.P(sy["cind"]), O.P(sy["val"]), 1, C.byref(A))
+    opts = S.senk_ilu_opts(S.SENK_ILU0 if kind == "ilu0" else S.SENK_ILUB, 0, 2, 2, 1 << S.SENK_FACTOR_F64, 1)
+    S.call("senk_prec_create_ilu", ctx.h, A, O.P(sy["rptr"]), O.P(sy["cind"]), O.P(sy["val"]), O.P(sy["cptr"]), sy["nc"],
+           8, C.byref(opts), C.byref(M))
+    db, dx, res = ctx.array(sy["x"]), ctx.zeros(N), S.senk_result()
+    o = S.solve_opts(solver=S.SENK_GMRES, m=30, eps=1e-8, max_iter=3000)
+    solve = lambda: S.lib().senk_solve(ctx.h, A, M, db.p, dx.p, C.byref(o), C.byref(res), None, 0)
+    try:
+        assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 1) == 0
+        S.call("senk_prec_apply_f64", M, db.p, dx.p)
+        assert S.lib().senk_prec_check(M) == 11 and S.lib().senk_prec_check(M) == 0
+        dx.zero()
+        assert solve() == 11
+        assert S.lib().senk_ctx_set_trsv_polls(ctx.h, 0) == 0
+        dx.zero()
+        assert solve() == 0 and res.converged == 1 and res.true_relres <= 1e-7
+        assert S.lib().senk_prec_check(M) == 0
+    finally:
+        S.lib().senk_ctx_set_trsv_polls(ctx.h, 0)
+        S.lib().senk_prec_destroy(M)
+        S.lib().senk_mat_destroy(A)
