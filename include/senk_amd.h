@@ -64,6 +64,13 @@ int senk_ctx_synchronize(senk_ctx ctx);
  * arrays polls (at least half a microsecond each) before it gives up and the solve's result
  * becomes invalid (SENK_ERR_TIMEOUT).  0 restores the default, 2^22. */
 int senk_ctx_set_trsv_polls(senk_ctx ctx, int polls);
+/* No reference counterpart: how the workgroups of those solves share out the rows.  0: by
+ * workgroup number, faster, for which no other kernel with waits between its workgroups may
+ * run on the device at the same time; 1: by tickets drawn in the order of arrival, which ends
+ * whatever runs beside it; -1, the default: 1 while another context of this process lives on
+ * the device, else 0.  A process that shares the device with another one that runs such solves
+ * sets 1 (with 0 the two could hold each other up until the waits give up).  Same bits. */
+int senk_ctx_set_trsv_tickets(senk_ctx ctx, int mode);
 int senk_device_count(int *count);
 int senk_device_malloc(senk_ctx ctx, size_t bytes, void **dptr);
 int senk_device_free(senk_ctx ctx, void *dptr);

@@ -71,6 +71,10 @@ int ctx_sweep_check(Ctx *c) {
     record_error("a single-launch triangular solve gave up a wait");
     return SENK_ERR_TIMEOUT;
 }
+DeviceContexts &device_contexts(int device) {
+    static DeviceContexts d[64];
+    return d[device & 63];
+}
 int ctx_work(Ctx *c, size_t bytes, void **out) { return arena_get(c->work, bytes, out); }
 int ctx_events(Ctx *c) {
     if (c->dring_h) return SENK_OK;
@@ -322,13 +326,22 @@ int senk_ctx_create(int device, senk_ctx *out) {
     SENK_HIP(hipHostMalloc((void **)&c.hpinned_i, sizeof(int) * 64, hipHostMallocDefault));
     SENK_HIP(hipHostMalloc((void **)&c.sweep_err, 64, hipHostMallocCoherent));
     *c.sweep_err = 0;
+    SENK_HIP(hipMalloc(&c.sweep_ticket, sizeof(unsigned)));
+    SENK_HIP(hipMemset(c.sweep_ticket, 0, sizeof(unsigned)));
     SENK_HIP(hipHostGetDevicePointer((void **)&c.sweep_err_d, c.sweep_err, 0));
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) c.num_cus = prop.multiProcessorCount;
     // the no-allocation entry point's scratch array on this device (once per device); a
     // failure here leaves every other entry point working and makes that one report it
     (void)noalloc_init(device);
-    SENK_HIP(hipDeviceSynchronize());
+    {
+        std::lock_guard<std::mutex> held(device_contexts(device).m);
+        device_contexts(device).n++;
+    }
+    // sweeps that another context launched while it was alone end before this one's begin
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) (void)senk_ctx_destroy(ctx);
+    SENK_HIP(e);
     *out = ctx;
     return SENK_OK;
 }
@@ -337,6 +350,10 @@ int senk_ctx_destroy(senk_ctx ctx) {
     Ctx &c = ctx->c;
     (void)hipSetDevice(c.device);
     (void)hipStreamSynchronize(c.stream);
+    {
+        std::lock_guard<std::mutex> held(device_contexts(c.device).m);
+        device_contexts(c.device).n--;
+    }
     if (c.work.p) (void)hipFree(c.work.p);
     if (c.outer.p) (void)hipFree(c.outer.p);
     for (hipEvent_t e : c.ev)
@@ -346,6 +363,7 @@ int senk_ctx_destroy(senk_ctx ctx) {
     (void)hipFree(c.dscalars);
     for (SweepVec &v : c.sweep.v)
         if (v.p) (void)hipFree(v.p);
+    (void)hipFree(c.sweep_ticket);
     (void)hipHostFree(c.sweep_err);
     (void)hipHostFree(c.hpinned);
     (void)hipHostFree(c.hpinned_i);
@@ -362,6 +380,12 @@ int senk_ctx_set_trsv_polls(senk_ctx ctx, int polls) {
     CTX_CHECK(ctx);
     if (polls < 0) return SENK_ERR_ARG;
     ctx->c.sweep_polls = polls ? std::min(polls, 1 << 29) : senk_amd::kSweepPolls;
+    return SENK_OK;
+}
+int senk_ctx_set_trsv_tickets(senk_ctx ctx, int mode) {
+    CTX_CHECK(ctx);
+    if (mode < -1 || mode > 1) return SENK_ERR_ARG;
+    ctx->c.sweep_tickets = mode;
     return SENK_OK;
 }
 int senk_device_malloc(senk_ctx ctx, size_t bytes, void **dptr) {
@@ -576,7 +600,7 @@ int senk_trsv_plan_create(senk_ctx ctx, const int *rptr, const int *cind, int N,
     p->s.seq_upper = upper != 0;
     int st = upload(ctx, &p->s.dblk, lists.data(), lists.size());
     p->s.dseq = p->s.dblk + blk.size();
-    p->s.dpos = p->s.dseq + (size_t)p->s.streams * p->s.seq_waves * 64;
+    p->s.dpos = p->s.dseq + (size_t)p->s.seq_waves * 64;
     if (st == SENK_OK && hipStreamSynchronize(ctx->c.stream) != hipSuccess) st = SENK_ERR_HIP;
     if (st != SENK_OK) {
         (void)senk_trsv_plan_destroy(p);

@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -73,9 +74,21 @@ struct Ctx {
     SweepVecs sweep;
     int sweep_polls = kSweepPolls;
     unsigned *sweep_err = nullptr, *sweep_err_d = nullptr;
+    // the counter their workgroups draw tickets from (device), its value once all launches so
+    // far are done, and when they do: 1 always, 0 never, -1 if another context lives on the device
+    unsigned *sweep_ticket = nullptr, sweep_base = 0;
+    int sweep_tickets = -1;
     unsigned sweep_tag = 0;  // number of the last such launch: what the word holds if it gave up
     unsigned dseq = 0;  // last sequence number handed out for the ring (runs on across solves)
 };
+// The contexts that live on a device; m is held while one is counted and while a kernel whose
+// progress depends on the count is launched.
+struct DeviceContexts {
+    std::mutex m;
+    int n = 0;
+};
+DeviceContexts &device_contexts(int device);
+
 // Creates the context's reusable events and pinned ring on first use.
 int ctx_events(Ctx *c);
 
@@ -97,9 +110,9 @@ struct Schedule {
     int nlev = 0;
     std::vector<int> lev_ptr;  // host
     int *dblk = nullptr;       // device, optional
-    // plans (bsize 1, dblk): the rows in the order of the single-launch solve, `streams`
-    // streams of `seq_waves` waves of 64 rows (device; -1: none) and each row's place in it,
-    // for upper = seq_upper solves
+    // plans (bsize 1, dblk): the rows in the order of the single-launch solve, `seq_waves`
+    // waves of 64 rows on `streams` XCDs (device; -1: none), and each row's place in it, for
+    // upper = seq_upper solves
     int *dseq = nullptr, *dpos = nullptr;
     int streams = 0, seq_waves = 0, max_ext = 0;  // max_ext: most off-diagonal entries of a row
     bool seq_upper = false;
@@ -213,7 +226,7 @@ template <typename T>
 int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rptr, const int *cind, const T *val,
                      const T *x, T *y, const double *in_scale, const int *stop, bool *done);
 // Rows blk of a level schedule (bsize 1) in the order of the single-launch solve: out = blk,
-// the sequence of streams * waves * 64 rows, and each row's place in it.
+// the sequence of waves * 64 rows, and each row's place in it.
 void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, int *streams, int *waves,
                     std::vector<int> &out);
 template <typename T>

@@ -8,18 +8,29 @@
 // resets the context's other vector to the sentinel for the next solve, so no fill kernel
 // runs.  x may alias y: only a row's own x is read, before its y is written.
 //
-// Workgroup b belongs to stream b mod 8, the XCD the dispatcher hands it to, and holds the
-// stream's ticket b / 8; stream x solves the x-th eighth of every level (in an ABMC order a
-// band of the domain), so most gathers are served by the XCD's own L2.  Progress: every
-// stream takes its rows level by level, so the unfinished row of the lowest level waits on
-// nothing unfinished, and the first unfinished workgroup of its stream, all earlier ones of
-// that XCD's dispatcher being finished, is resident or next.  Any other order ends in the
-// bounded poll, which raises the context's time-out word, not in a hang.
+// A launch's workgroups are numbered by ticket, 0, 1, ...: ticket 8 j + x solves part j of
+// stream x, the x-th eighth of every level (in an ABMC order a band of the domain), level by
+// level.  Two ways to number them:
+//  - by workgroup number (a context that is alone on its device): ticket b runs on the XCD that
+//    the dispatcher hands workgroup b to, b mod 8, so most gathers are served by the XCD's own
+//    L2.  Progress needs every dispatcher to hand out its workgroups in increasing order and
+//    no other waiting kernel beside this one: the unfinished row of the lowest level then waits
+//    on nothing unfinished, and its workgroup is resident or next.
+//  - drawn from the context's counter in the order of arrival (SweepWait::ticket), as soon as
+//    another context lives on the device: its waiting workgroups could fill one XCD and ours
+//    another, each waiting for a workgroup that finds no room where the other waits.  A drawn
+//    ticket waits on lower tickets only (in a plan: see k_csr_rows), which are drawn too and
+//    running or done, so a launch ends whatever runs beside it and however they arrive.  The draws
+//    cost 10-15 ns each, all on one address: 64^3 grid, blocks of 8, GMRES(30) 25.8 -> 31.8
+//    ms; 61x64x67 plans 557 -> 673 us; block solve of 45^3 elasticity 151 -> 161 us.
+// Any other order ends in the bounded poll, which raises the context's time-out word, not in a
+// hang.
 //
 // Per row the operations and their order are the sequential solve's: the same bits.
 #include "sweep.hpp"
 
 #include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 namespace senk_amd {
@@ -34,9 +45,12 @@ struct SweepLevels {
 // What a launch's waits need: the context's time-out word, the launch's number, which a wait
 // that gives up writes there, and the polls after which it does.  The other waits of the
 // launch then give up as well; those of later launches, whatever the word still holds, do not.
+// ticket: the counter that the workgroups draw from and its value before the launch (null:
+// tickets are workgroup numbers).
 struct SweepWait {
     unsigned *err, tag;
     int limit;
+    unsigned *ticket, base;
 };
 
 namespace {
@@ -82,6 +96,21 @@ __device__ __forceinline__ void await_rows(const T *z, const int (&cc)[CH], cons
             if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
         b = __ballot(want >= 0);
     }
+}
+
+// The ticket of workgroup `number` of the `n` that solve; -1: the counter is out of step with
+// the host's count (the launch then reports a time-out).
+__device__ __forceinline__ int draw_ticket(const SweepWait &wt, int number, int n) {
+    if (!wt.ticket) return number;
+    __shared__ int tk;
+    if (threadIdx.x == 0) {
+        const unsigned t =
+            __hip_atomic_fetch_add(wt.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - wt.base;
+        tk = t < (unsigned)n ? (int)t : -1;
+        if (tk < 0) __hip_atomic_store(wt.err, wt.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(tk);
 }
 
 // Level of ticket j (uniform): the last l with ticket[l] <= j.
@@ -208,7 +237,9 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, co
                                                               SweepWait wt, const int *__restrict__ stop) {
     __shared__ T sv[kCsrWaves][kCsrCap<T>];
     __shared__ int sc[kCsrWaves][kCsrCap<T>];
-    const int xs = (int)(blockIdx.x % kXcds), j = (int)(blockIdx.x / kXcds);
+    const int tk = draw_ticket(wt, (int)blockIdx.x, (int)gridDim.x);
+    if (tk < 0) return;
+    const int xs = tk % kXcds, j = tk / kXcds;
     const int l = level_of(lv, j), sl = __builtin_amdgcn_readfirstlane(band_slice(lv, l, j, xs, 64));
     if (sl < 0) return;
     const int wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
@@ -260,11 +291,14 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, co
 }
 
 // ------------------------------------------------------------------ CSR, planned (level lists)
-// Rows of a level schedule (bsize 1): seq holds the rows in stream order, wave w of stream x
-// taking seq[(w * streams + x) * 64 + lane] (-1: none).  Rows of several levels may share a
-// wave, so no lane waits for another: every lane polls for its own entries, and a lane whose
-// round is complete subtracts it and goes on or publishes its row, whatever the others wait
-// for.  Rows are published by their place in seq (pos), not by row: the rows that a level's
+// Rows of a level schedule (bsize 1): ticket t takes the rows seq[64 t + lane] (-1: none).
+// Rows of several levels may share a wave, so no lane waits for another: every lane polls for
+// its own entries, and a lane whose round is complete subtracts it and goes on or publishes its
+// row, whatever the others wait for.  A wave's rows are 64 consecutive ones of one stream, and a
+// ticket's begin at most one wave of its stream past the level in which a higher ticket's begin.
+// So of the waves that have drawn a ticket, at most two a stream cannot finish before one that
+// has not drawn: they fill no XCD, and the next workgroup finds room.
+// Rows are published by their place in seq (pos), not by row: the rows that a level's
 // consecutive rows wait for are then close together, and a poll touches a few lines instead
 // of one per entry (published by row, every resident wave's polls kept the memory system
 // busy: 61x64x67 7-point grid, 190 levels, L + U in FP64 1352 us, 581 by place; one launch
@@ -272,16 +306,18 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_csr_sweep(SweepLevels lv, co
 // with the sentinel by the CU's own cache (every other poll plain 581 us, none 551; 27-point
 // 38^3 1332 and 1249).  What is left is one publish-and-poll round trip per level, about 1.45 us.
 template <typename T, bool UPPER, int CH>
-__global__ __launch_bounds__(64) void k_csr_rows(int streams, const int *__restrict__ seq,
+__global__ __launch_bounds__(64) void k_csr_rows(int waves, int xcds, const int *__restrict__ seq,
                                                  const int *__restrict__ pos,
                                                  const int *__restrict__ rptr, const int *__restrict__ cind,
                                                  const T *__restrict__ val, const T *x, T *y, T *z, T *reset,
                                                  const double *__restrict__ in_scale, SweepWait wt,
                                                  const int *__restrict__ stop) {
     using U = typename Bits<T>::U;
-    const int xs = (int)(blockIdx.x % kXcds), w = (int)(blockIdx.x / kXcds);
-    if (xs >= streams) return;
-    const int mine = (w * streams + xs) * 64 + (int)(threadIdx.x & 63);
+    const int xcd = (int)(blockIdx.x % kXcds), number = (int)(blockIdx.x / kXcds) * xcds + xcd;
+    if (xcd >= xcds) return;
+    const int tk = draw_ticket(wt, number, waves);
+    if (tk < 0) return;
+    const int mine = tk * 64 + (int)(threadIdx.x & 63);
     const int row = seq[mine];
     const int stopped = stop ? *stop : 0;
     bool act = row >= 0;
@@ -385,7 +421,9 @@ __global__ __launch_bounds__(64 * kCsrWaves) void k_bcsr_sweep(
     constexpr int QB = BNW == 1 ? 8 : 4;                    // in-part blocks held in LDS
     __shared__ int qc[kCsrWaves][QB][64];
     __shared__ T qv[kCsrWaves][QB][BNW][64];
-    const int xs = (int)(blockIdx.x % kXcds), j = (int)(blockIdx.x / kXcds);
+    const int tk = draw_ticket(wt, (int)blockIdx.x, (int)gridDim.x);
+    if (tk < 0) return;
+    const int xs = tk % kXcds, j = tk / kXcds;
     const int l = level_of(lv, j), sl = __builtin_amdgcn_readfirstlane(band_slice(lv, l, j, xs, bpw));
     if (sl < 0) return;
     const int lane = (int)(threadIdx.x & 63), wv = (int)(threadIdx.x >> 6);
@@ -581,7 +619,7 @@ __global__ __launch_bounds__(kBlock) void k_fill_sentinel2(size_t n, T *p) {
 // ------------------------------------------------------------------ host side
 // The sweep vectors of the next solve of n rows: *z all-sentinel (filled here where the
 // last solves left less than that), *reset the vector the launch must fill in its first n
-// rows; sweep_launched follows the launch.  false: no memory (the caller takes its
+// rows; SweepLaunch::done follows the launch.  false: no memory (the caller takes its
 // launch-per-level path).
 template <typename T>
 static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
@@ -627,22 +665,35 @@ static int sweep_vectors(Ctx *c, size_t n, T **z, T **reset, bool *ok) {
     *ok = true;
     return SENK_OK;
 }
-static SweepWait sweep_wait(Ctx *c) {
-    if (++c->sweep_tag == 0) c->sweep_tag = 1;  // 0: nothing gave up
-    return SweepWait{c->sweep_err_d, c->sweep_tag, c->sweep_polls};
-}
-// The status of the launch that took the vectors of sweep_vectors<T>(n).
-template <typename T>
-static int sweep_launched(Ctx *c, size_t n) {
-    const hipError_t e = hipGetLastError();
-    if (e == hipSuccess) {
-        c->sweep.solved(n, (int)sizeof(T));
+// Held while a sweep is launched: which way its tickets are numbered depends on the contexts
+// that live on the device, and senk_ctx_create waits, once its own is counted, for what was
+// launched under the former count.
+struct SweepLaunch {
+    Ctx *c;
+    std::lock_guard<std::mutex> held;
+    SweepWait wt;
+    explicit SweepLaunch(Ctx *ctx) : c(ctx), held(device_contexts(ctx->device).m) {
+        if (++c->sweep_tag == 0) c->sweep_tag = 1;  // 0: nothing gave up
+        const bool draw = c->sweep_tickets < 0 ? device_contexts(c->device).n > 1 : c->sweep_tickets != 0;
+        wt = SweepWait{c->sweep_err_d, c->sweep_tag, c->sweep_polls, draw ? c->sweep_ticket : nullptr, c->sweep_base};
+    }
+    // The status of the launch, which took the vectors of sweep_vectors<T>(n) and whose `tickets`
+    // workgroups solve.
+    template <typename T>
+    int done(size_t n, int tickets) {
+        const hipError_t e = hipGetLastError();
+        if (e == hipSuccess) {
+            c->sweep.solved(n, (int)sizeof(T));
+            if (wt.ticket) c->sweep_base += (unsigned)tickets;
+            return SENK_OK;
+        }
+        c->sweep.spoiled();
+        (void)hipMemsetAsync(c->sweep_ticket, 0, sizeof(unsigned), c->stream);
+        c->sweep_base = 0;
+        SENK_HIP(e);
         return SENK_OK;
     }
-    c->sweep.spoiled();
-    SENK_HIP(e);
-    return SENK_OK;
-}
+};
 
 // Average rows per level below which a plan's rows go through one stream, i.e. one XCD: a
 // thin level has no use for the others' bandwidth, and its waits stay on one die.  L + U in
@@ -654,29 +705,49 @@ void sweep_sequence(const Schedule &s, const std::vector<int> &blk, bool upper, 
                     std::vector<int> &out) {
     const size_t n = blk.size();
     const int S = s.nlev > 0 && (double)n / s.nlev < kPlanOneStream ? 1 : kXcds;
-    size_t len[kXcds] = {};
-    for (int l = 0; l < s.nlev; l++) {
-        const long long k = s.lev_ptr[l + 1] - s.lev_ptr[l];
-        for (int x = 0; x < S; x++) len[x] += (size_t)(k * (x + 1) / S - k * x / S);
-    }
-    size_t w = 0;
-    for (int x = 0; x < S; x++) w = std::max(w, (len[x] + 63) / 64);
-    *streams = S;
-    *waves = (int)w;
-    // blk, then the sequence, then each row's place in it
-    out.assign(n + w * S * 64 + n, -1);
-    std::copy(blk.begin(), blk.end(), out.begin());
-    int *seq = out.data() + n, *pos = seq + w * S * 64;
-    size_t at[kXcds] = {};
+    // the rows of every stream, level by level, and the level of every wave's first row
+    std::vector<int> row[kXcds], first[kXcds];
     for (int step = 0; step < s.nlev; step++) {
         const int l = upper ? s.nlev - 1 - step : step;
         const long long a = s.lev_ptr[l], k = s.lev_ptr[l + 1] - a;
         for (int x = 0; x < S; x++)
             for (long long i = a + k * x / S; i < a + k * (x + 1) / S; i++) {
-                const size_t q = at[x]++, p = ((q / 64) * S + x) * 64 + q % 64;
-                seq[p] = blk[i];
-                pos[blk[i]] = (int)p;
+                if (row[x].size() % 64 == 0) first[x].push_back(step);
+                row[x].push_back(blk[i]);
             }
+    }
+    // Rounds of one wave a stream.  A stream whose next wave begins in a later level than another
+    // stream's passes (an empty wave), unless its last one does not: it is at most one ahead.
+    std::vector<int> order[kXcds];  // wave of the stream per round, or -1
+    size_t at[kXcds] = {};
+    for (;;) {
+        int low = s.nlev;
+        for (int x = 0; x < S; x++)
+            if (at[x] < first[x].size()) low = std::min(low, first[x][at[x]]);
+        if (low == s.nlev) break;
+        for (int x = 0; x < S; x++) {
+            const size_t i = at[x];
+            const bool take = i < first[x].size() && (first[x][i] <= low || i == 0 || first[x][i - 1] <= low);
+            order[x].push_back(take ? (int)i : -1);
+            at[x] += take;
+        }
+    }
+    const size_t w = order[0].size() * S;
+    *streams = S;
+    *waves = (int)w;
+    // blk, then the sequence, then each row's place in it
+    out.assign(n + w * 64 + n, -1);
+    std::copy(blk.begin(), blk.end(), out.begin());
+    int *seq = out.data() + n, *pos = seq + w * 64;
+    for (size_t t = 0; t < w; t++) {
+        const std::vector<int> &r = row[t % S];
+        const int k = order[t % S][t / S];
+        if (k < 0) continue;
+        for (size_t i = (size_t)k * 64; i < std::min(r.size(), (size_t)k * 64 + 64); i++) {
+            const size_t p = t * 64 + i % 64;
+            seq[p] = r[i];
+            pos[r[i]] = (int)p;
+        }
     }
 }
 
@@ -716,22 +787,23 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
     T *z = nullptr, *reset = nullptr;
     if (s.dblk) {
         if (BS != 1 || !s.dseq || !s.dpos || s.seq_upper != upper) return SENK_OK;
-        const size_t nz = (size_t)s.seq_waves * s.streams * 64;
+        const size_t nz = (size_t)s.seq_waves * 64;
         bool ok = false;
         SENK_TRY(sweep_vectors<T>(c, nz, &z, &reset, &ok));
         if (!ok) return SENK_OK;
-        const int grid = kXcds * s.seq_waves;
+        const int grid = s.seq_waves / s.streams * kXcds;
+        SweepLaunch sl(c);
         // rounds of 4 where no row has more entries, else of 16: a second round costs its own
         // chain of dependent loads after the last row of the first is there
 #define SENK_CSR_ROWS(UP, CH)                                                                                      \
-    k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.streams, s.dseq, s.dpos, rptr, cind, val, x, y, z, reset, \
-                                                      UP ? nullptr : in_scale, sweep_wait(c), stop)
+    k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.seq_waves, s.streams, s.dseq, s.dpos, rptr, cind, val, x, y, z, reset, \
+                                                      UP ? nullptr : in_scale, sl.wt, stop)
         if (upper && s.max_ext <= 4) SENK_CSR_ROWS(true, 4);
         else if (upper) SENK_CSR_ROWS(true, 16);
         else if (s.max_ext <= 4) SENK_CSR_ROWS(false, 4);
         else SENK_CSR_ROWS(false, 16);
 #undef SENK_CSR_ROWS
-        SENK_TRY(sweep_launched<T>(c, nz));
+        SENK_TRY(sl.done<T>(nz, s.seq_waves));
         *done = true;
         return SENK_OK;
     }
@@ -742,14 +814,15 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
     SENK_TRY(sweep_vectors<T>(c, (size_t)N, &z, &reset, &ok));
     if (!ok) return SENK_OK;
     const int grid = kXcds * tickets;
+    SweepLaunch sl(c);
 #define SENK_CSR_SWEEP(B)                                                                                        \
     case B:                                                                                                      \
         if (upper)                                                                                               \
             k_csr_sweep<T, B, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z, reset, \
-                                                                            nullptr, sweep_wait(c), stop);      \
+                                                                            nullptr, sl.wt, stop);              \
         else                                                                                                     \
             k_csr_sweep<T, B, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(lv, rptr, cind, val, x, y, z,       \
-                                                                             reset, in_scale, sweep_wait(c),    \
+                                                                             reset, in_scale, sl.wt,             \
                                                                              stop);                              \
         break;
     switch (BS) {
@@ -763,7 +836,7 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
         default: return SENK_ERR_UNSUPPORTED;  // not reached: BS divides 64
     }
 #undef SENK_CSR_SWEEP
-    SENK_TRY(sweep_launched<T>(c, (size_t)N));
+    SENK_TRY(sl.done<T>((size_t)N, kXcds * tickets));
     *done = true;
     return SENK_OK;
 }
@@ -773,15 +846,15 @@ template int launch_csr_sweep<float>(Ctx *, const Schedule &, bool, int, const i
                                      const float *, float *, const double *, const int *, bool *);
 
 template <typename T, int BNL, int BNW>
-static void bcsr_sweep(Ctx *c, const SweepLevels &lv, int tickets, const Schedule &s, bool upper, int part, int bpw,
+static void bcsr_sweep(Ctx *c, const SweepWait &wt, const SweepLevels &lv, int tickets, const Schedule &s, bool upper, int part, int bpw,
                        const int *brptr, const int *bcind, const T *bval, const T *x, T *y, T *z, T *reset) {
     const int grid = kXcds * tickets;
     if (upper)
         k_bcsr_sweep<T, BNL, BNW, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
-            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, sweep_wait(c));
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, wt);
     else
         k_bcsr_sweep<T, BNL, BNW, false><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
-            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, sweep_wait(c));
+            lv, s.dblk, s.bsize, part, bpw, brptr, bcind, bval, x, y, z, reset, wt);
 }
 template <typename T>
 int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,
@@ -818,8 +891,9 @@ int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int
     bool ok = false;
     SENK_TRY(sweep_vectors<T>(c, (size_t)N, &z, &reset, &ok));
     if (!ok) return SENK_OK;
-    launch(c, lv, tickets, s, upper, part, bpw, brptr, bcind, bval, x, y, z, reset);
-    SENK_TRY(sweep_launched<T>(c, (size_t)N));
+    SweepLaunch sl(c);
+    launch(c, sl.wt, lv, tickets, s, upper, part, bpw, brptr, bcind, bval, x, y, z, reset);
+    SENK_TRY(sl.done<T>((size_t)N, kXcds * tickets));
     *done = true;
     return SENK_OK;
 }

@@ -80,6 +80,16 @@ def _tridiagonal(n):
     return rptr.astype(np.int32), cols[o].astype(np.int32), vals[o]
 
 
+def _chain_then_wide(chain, wide):
+    """`chain` levels of one row, then one of `wide` rows that wait for the last of them: on all
+    XCDs, most of whose streams have nothing in the chain's levels."""
+    rows = [[i - 1, i] if 0 < i < chain else [i] if i == 0 else [chain - 1, i] for i in range(chain + wide)]
+    rptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    cind = np.concatenate(rows).astype(np.int32)
+    val = np.where(cind == np.repeat(np.arange(len(rows)), np.diff(rptr)), 3.0, -1.0)
+    return rptr, cind, val
+
+
 # sizes around the slice of 64 rows and the ticket of 4 slices, rows of more than one round of
 # gathers, slices of more entries than the wave stages in LDS (27-point in FP64)
 @pytest.mark.parametrize("bsize", [1, 2, 4, 8, 16, 32, 64])
@@ -345,3 +355,60 @@ def test_handles_without_the_sliced_layout_report_a_wait_given_up(ctx, kind):
         S.lib().senk_ctx_set_trsv_polls(ctx.h, 0)
         S.lib().senk_prec_destroy(M)
         S.lib().senk_mat_destroy(A)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_tickets_by_number_and_by_arrival(ctx, mode):
+    """Both ways of sharing out the rows give the sequential solve's bits, in any turn with the
+    other (the counter's base moves with the launches that draw)."""
+    assert S.lib().senk_ctx_set_trsv_tickets(ctx.h, 2) == 1
+    try:
+        for k, (bsize, dt) in enumerate([(1, np.float64), (8, np.float32), (64, np.float64)]):
+            assert S.lib().senk_ctx_set_trsv_tickets(ctx.h, mode if k != 1 else 1 - mode) == 0
+            _abmc_case(ctx, S.gen_convdiff27(11, 10.0), bsize, "connect", dt)
+            _plan_case(ctx, S.gen_poisson7(9, 13, 5), dt)       # one XCD
+            _plan_case(ctx, S.gen_poisson7(48, 46, 47), dt)     # all
+            _plan_case(ctx, _tridiagonal(200), dt)
+            _plan_case(ctx, _chain_then_wide(150, 150000), dt)
+            t, u, yl, yu = _bcsr(ctx, 9, 3, 3, (24, 48, 96)[k])
+            assert np.array_equal(t, yl) and np.array_equal(u, yu)
+    finally:
+        S.lib().senk_ctx_set_trsv_tickets(ctx.h, -1)
+
+
+def test_solves_of_two_contexts_at_once(ctx):
+    """Two contexts' solves in flight together, 8 streams of rows each, with neither waiting for
+    the other on the host."""
+    rptr, cind, val = S.gen_poisson7(48, 46, 47)
+    N = len(rptr) - 1
+    sy = abmc_system(rptr, cind, val, 1)
+    L, U = ilu_factors(sy)
+    x = np.random.default_rng(6).uniform(-1, 1, N)
+    yl, yu = _seq(L, U, x)
+    other = S.Context(0)
+    try:
+        runs = []
+        for c in (ctx, other):
+            d = [c.array(t) for t in (*L, *U, x)]
+            plans = []
+            for f, up in ((L, 0), (U, 1)):
+                p = C.c_void_p()
+                S.call("senk_trsv_plan_create", c.h, O.P(f[2]), O.P(f[1]), N, up, C.byref(p))
+                plans.append(p)
+            runs.append((c, d, plans, [c.zeros(N) for _ in range(2)]))
+        for k in range(12):
+            for c, d, plans, (a, b) in runs:
+                if k % 3 == 2:
+                    cp = O.P(sy["cptr"])
+                    S.call("senk_sptrsv_csr_l_abmc_f64", c.h, *(t.p for t in d[:3]), d[6].p, a.p, N, cp, sy["nc"], 1)
+                    S.call("senk_sptrsv_csr_u_abmc_f64", c.h, *(t.p for t in d[3:6]), a.p, b.p, N, cp, sy["nc"], 1)
+                else:
+                    S.call("senk_sptrsv_csr_l_f64", c.h, plans[0], *(t.p for t in d[:3]), d[6].p, a.p, N)
+                    S.call("senk_sptrsv_csr_u_f64", c.h, plans[1], *(t.p for t in d[3:6]), a.p, b.p, N)
+        for c, d, plans, (a, b) in runs:
+            assert np.array_equal(a.download(), yl) and np.array_equal(b.download(), yu)
+            for p in plans:
+                S.lib().senk_trsv_plan_destroy(p)
+        del runs, d, a, b
+    finally:
+        other.close()
