@@ -243,7 +243,8 @@ __device__ __forceinline__ SliceHead<V, BS> slice_head(int slice, const int4 *__
     return h;
 }
 
-template <typename T, typename V, int BS, bool UPPER, bool SWEEP, int CH = 8, bool PIPE = false, bool O32 = false>
+template <typename T, typename V, int BS, bool UPPER, bool SWEEP, int CH = 8, bool PIPE = false, bool O32 = false,
+          bool ALL = false>
 __device__ __forceinline__ void solve_slice_body(const SliceHead<V, BS> &h, const int *__restrict__ blk_list,
                                                  const int *__restrict__ scol, const V *__restrict__ ve,
                                                  const V *__restrict__ vi, const T *x, T *y,
@@ -340,32 +341,54 @@ __device__ __forceinline__ void solve_slice_body(const SliceHead<V, BS> &h, cons
             // While it waits the wave polls one row only, the last one still missing of its first
             // waiting lane (the latest level); when that one is there it reads all the missing
             // ones again.  With every missing row polled by every waiting wave (and a sleep
-            // between polls) the polls themselves slowed the rows waited for down: FP32
-            // application, 7-point 96^3 connect blocks of 8, 75.8 -> 56.3 us; FP64, 27-point 71^3
-            // blocks of 16, 131.8 -> 108.7 us, unstructured 300,000 rows 550 -> 485 us; two
-            // colors (128^3 simple blocks of 8) unchanged.
-            int want = -1;
+            // between polls: ALL, where launch_xticket still takes it) the polls themselves slowed
+            // the rows waited for down: FP32 application, 7-point 96^3 connect blocks of 8, 75.8 ->
+            // 56.3 us; FP64, 27-point 71^3 blocks of 16, 131.8 -> 108.7 us, unstructured 300,000
+            // rows 550 -> 485 us.  Where the rows of a level end together the second read is a
+            // round trip more: 27-point systems of 32^3 to 48^3 in 8 colors of whole lines (simple
+            // blocks of 8) lose 3%, those whose lines the blocks cut gain 8-13%.
+            if constexpr (ALL) {
+                bool pend = false;
 #pragma unroll
-            for (int q = 0; q < CH; q++)
-                if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
-            unsigned long long miss = __ballot(want >= 0);
-            for (int spin = 0; miss;) {
-                const T *p = ixp<O32>(y, __builtin_amdgcn_readlane(want, __ffsll((long long)miss) - 1));
-                while (load_agent(p) == Bits<T>::kSentinel && spin < kSweepSpinLimit) {
-                    spin++;
-                }
-                if (spin >= kSweepSpinLimit) {
-                    __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
+                for (int q = 0; q < CH; q++) pend |= on[q] && yb[q] == Bits<T>::kSentinel;
+                for (int spin = 0; __ballot(pend); spin++) {
+                    if (spin >= kSweepSpinLimit) {
+                        if (pend) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(2);
+                    pend = false;
 #pragma unroll
-                for (int q = 0; q < CH; q++)
-                    if (on[q] && yb[q] == Bits<T>::kSentinel) yb[q] = load_agent(ixp<O32>(y, cc[q]));
-                want = -1;
+                    for (int q = 0; q < CH; q++)
+                        if (on[q] && yb[q] == Bits<T>::kSentinel) {
+                            yb[q] = load_agent(ixp<O32>(y, cc[q]));
+                            pend |= yb[q] == Bits<T>::kSentinel;
+                        }
+                }
+            } else {
+                int want = -1;
 #pragma unroll
                 for (int q = 0; q < CH; q++)
                     if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
-                miss = __ballot(want >= 0);
+                unsigned long long miss = __ballot(want >= 0);
+                for (int spin = 0; miss;) {
+                    const T *p = ixp<O32>(y, __builtin_amdgcn_readlane(want, __ffsll((long long)miss) - 1));
+                    while (load_agent(p) == Bits<T>::kSentinel && spin < kSweepSpinLimit) {
+                        spin++;
+                    }
+                    if (spin >= kSweepSpinLimit) {
+                        __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        break;
+                    }
+#pragma unroll
+                    for (int q = 0; q < CH; q++)
+                        if (on[q] && yb[q] == Bits<T>::kSentinel) yb[q] = load_agent(ixp<O32>(y, cc[q]));
+                    want = -1;
+#pragma unroll
+                    for (int q = 0; q < CH; q++)
+                        if (on[q] && yb[q] == Bits<T>::kSentinel) want = cc[q];
+                    miss = __ballot(want >= 0);
+                }
             }
 #pragma unroll
             for (int q = 0; q < CH; q++) yv[q] = __builtin_bit_cast(T, yb[q]);
@@ -557,7 +580,7 @@ __global__ __launch_bounds__(64 * kTicketWaves) void k_sptrsv_ticket(
 // ticket j of stream x solves slice 64 j + 8 x + w: the wave goes from its workgroup
 // number to its slice descriptor and row words without a lookup.  Otherwise
 // xslice[x][j][w] names the slice (-1: none).
-template <typename T, typename V, int BS, bool UPPER, int CH, bool PIPE, bool O32>
+template <typename T, typename V, int BS, bool UPPER, int CH, bool PIPE, bool O32, bool ALL>
 __global__ __launch_bounds__(64 * kXTicketWaves) void k_sptrsv_xticket(
     int xwg, const int *__restrict__ xslice, const int4 *__restrict__ sinfo, const int *__restrict__ blk_list,
     const typename RowWord<BS>::W *__restrict__ rw, const int *__restrict__ next, const int *__restrict__ scol,
@@ -574,7 +597,7 @@ __global__ __launch_bounds__(64 * kXTicketWaves) void k_sptrsv_xticket(
     const int stopped = stop_flag ? *stop_flag : 0;
     const SliceHead<V, BS> h = slice_head<V, BS, UPPER, O32>(slice, sinfo, rw, next, dinv, sx);
     if (stopped) return;
-    solve_slice_body<T, V, BS, UPPER, true, CH, PIPE, O32>(h, blk_list, scol, ve, vi, x, y, in_scale, reset,
+    solve_slice_body<T, V, BS, UPPER, true, CH, PIPE, O32, ALL>(h, blk_list, scol, ve, vi, x, y, in_scale, reset,
                                                            sync + kSweepErr, copy, ep_a, ep_b, pre);
 }
 
@@ -728,28 +751,48 @@ int launch_xticket(Ctx *c, const Schedule &s, TriLayout &L, const V *ve, const V
     // a second round: 72.3 against 62.9 us in the connect order.
     const bool ch4 = std::is_same<T, double>::value && L.max_ext <= 8;
     const bool pipe = L.max_ext > (ch4 ? 4 : 8);
+    // Every missing row polled instead of one (solve_slice_body) where an average level has more
+    // slices than the line below, about half of the waves that are resident at once: there is then
+    // little to wait for, and the one-row wait, whose registers cost these kernels a wave per SIMD
+    // (FP64 8 -> 7 or 7 -> 6, FP32 with PIPE 6 -> 5), loses.  One row / all, us, with the slices
+    // per CU of a level: FP64 7-point simple blocks of 4, 72^3 (11.4) 15.7 / 15.5, 76^3 (13.4)
+    // 17.6 / 16.8, 80^3 (15.6) 19.2 / 17.6, 128^3 (64) 63.6 / 60.5; blocks of 8, 1000 x 800 (24)
+    // equal; FP32 27-point simple blocks of 16, 96^3 (6.8) 64.7 / 67.5, 112^3 (10.7) 91.0 / 88.8,
+    // 128^3 (16) 127.8 / 119.0.  The other kernels keep their waves and run the same either way.
+    const bool all = (ch4 || (std::is_same<T, float>::value && pipe)) && L.max_ext <= 32 &&
+                     (long long)L.nslices > (ch4 ? 13LL : 10LL) * c->num_cus * L.nsteps;
     // 32-bit byte offsets where every array the sweep indexes fits them (elements of at most
     // 8 bytes; the slice descriptors, 16 bytes each, number at most a 64th of the slots)
     const long long most = std::max({(long long)L.n, L.n_ext, L.n_int, (long long)L.nslices * 64});
     const bool o32 = most * 8 < (1LL << 32);
-#define SENK_XT_LAUNCH1(CHV, PIPEV, O32V)                                                                      \
-    k_sptrsv_xticket<T, V, BS, UPPER, CHV, PIPEV, O32V><<<kXcds * L.xwg, 64 * kXTicketWaves, 0, c->stream>>>(  \
+#define SENK_XT_LAUNCH1(CHV, PIPEV, O32V, ALLV)                                                                \
+    k_sptrsv_xticket<T, V, BS, UPPER, CHV, PIPEV, O32V, ALLV><<<kXcds * L.xwg, 64 * kXTicketWaves, 0, c->stream>>>(  \
         L.xwg, L.xslice, L.sinfo, s.dblk, (const W *)L.rw, L.next, L.scol, ve, vi, dinv, sx, x, y,              \
         UPPER ? nullptr : in_scale, reset, L.sync, copy, ep_a, ep_b, stop, pre)
-#define SENK_XT_LAUNCH(CHV, PIPEV)              \
-    do {                                        \
-        if (o32) SENK_XT_LAUNCH1(CHV, PIPEV, true);  \
-        else SENK_XT_LAUNCH1(CHV, PIPEV, false); \
+#define SENK_XT_LAUNCH(CHV, PIPEV, ALLV)                   \
+    do {                                                   \
+        if (o32) SENK_XT_LAUNCH1(CHV, PIPEV, true, ALLV);  \
+        else SENK_XT_LAUNCH1(CHV, PIPEV, false, ALLV);     \
     } while (0)
     // rows of more than 32 external entries (an irregular matrix's long tail): rounds of 16,
     // at 108-161 VGPRs, as the longest row of a level sets its time (unstructured n = 2^22,
     // blocks of 16: FP32 / FP64 application 944 / 1048 us against 1150 / 1260 us with rounds
     // of 8; the 27-point system, rows of 17-32, loses with them: FP64 315 against 246 us)
-    if (ch4 && pipe) SENK_XT_LAUNCH(4, true);
-    else if (ch4) SENK_XT_LAUNCH(4, false);
-    else if (L.max_ext > 32) SENK_XT_LAUNCH(16, true);
-    else if (pipe) SENK_XT_LAUNCH(8, true);
-    else SENK_XT_LAUNCH(8, false);
+    if (all) {
+        if constexpr (std::is_same<V, double>::value) {
+            if (pipe) SENK_XT_LAUNCH(4, true, true);
+            else SENK_XT_LAUNCH(4, false, true);
+        } else {
+            SENK_XT_LAUNCH(8, true, true);
+        }
+        SENK_LAUNCH_CHECK();
+        return SENK_OK;
+    }
+    if (ch4 && pipe) SENK_XT_LAUNCH(4, true, false);
+    else if (ch4) SENK_XT_LAUNCH(4, false, false);
+    else if (L.max_ext > 32) SENK_XT_LAUNCH(16, true, false);
+    else if (pipe) SENK_XT_LAUNCH(8, true, false);
+    else SENK_XT_LAUNCH(8, false, false);
 #undef SENK_XT_LAUNCH
 #undef SENK_XT_LAUNCH1
     SENK_LAUNCH_CHECK();

@@ -151,6 +151,25 @@ def test_layout_abmc_unstructured_long_rows(ctx):
     _check(ctx, sy, S.SENK_ILU0, 0, 16, colors=True)
 
 
+# levels of 3400 slices, above the lines from which a wait polls all of its rows: FP64 rows of one
+# round of gathers (4) and of two (6), FP32 rows of two (12)
+@pytest.mark.parametrize("k,bsize", [(4, 8), (6, 1), (12, 8)])
+def test_layout_two_large_levels(ctx, k, bsize):
+    half = 3400 * 64
+    rng = np.random.default_rng(k)
+    other = (np.arange(half)[:, None] + np.sort(rng.choice(1000, k, replace=False))[None, :] - 500) % half
+    other.sort(axis=1)
+    diag = np.arange(half)[:, None]
+    cind = np.concatenate([np.concatenate([diag, other + half], 1), np.concatenate([other, diag + half], 1)])
+    val = rng.uniform(-1, 1, cind.shape)
+    val[:half, 0] += 2 * k
+    val[half:, k] += 2 * k
+    sy = dict(N=2 * half, val=val.ravel(), cind=cind.ravel().astype(np.int32),
+              rptr=(np.arange(2 * half + 1) * (k + 1)).astype(np.int32), nc=2,
+              cptr=np.array([0, half // bsize, 2 * half // bsize], np.int32))
+    _check(ctx, sy, S.SENK_ILU0, 0, bsize, True)
+
+
 @pytest.mark.parametrize("p,bsize", [(1, 8), (2, 4)])
 def test_layout_ilup_fill(ctx, p, bsize):
     # ILU(p) fill can couple blocks of one color: the handle falls back to the
