@@ -881,7 +881,6 @@ static int ilu0_impl(senk_ctx ctx, T *dval, const int *dcind, const int *drptr, 
     int st = ctx_work(c, ((size_t)N + 1) * sizeof(int), &buf);
     int *dpos = static_cast<int *>(buf), *derr = dpos + N;
     if (!st && hipMemsetAsync(derr, 0, sizeof(int), c->stream) != hipSuccess) st = SENK_ERR_HIP;
-    if (!st) st = launch_find_diag(c, N, drptr, dcind, dpos);
     if (!st) st = launch_ilu0<T>(c, s, N, drptr, dcind, dpos, dval, derr);
     int *herr_p = c->hpinned_i + 2;
     if (!st && hipMemcpyAsync(herr_p, derr, sizeof(int), hipMemcpyDeviceToHost, c->stream) != hipSuccess)
@@ -1560,7 +1559,6 @@ int senk_prec_create_ilu(senk_ctx ctx, senk_mat A, const int *rptr, const int *c
         if ((st = dalloc(&dpos, (size_t)N))) break;
         if ((st = dalloc(&derr, 1))) break;
         if (hipMemsetAsync(derr, 0, sizeof(int), c->stream) != hipSuccess) { st = SENK_ERR_HIP; break; }
-        if ((st = launch_find_diag(c, N, dfr, dfc, dpos))) break;
         if ((st = launch_ilu0<double>(c, v.ls, N, dfr, dfc, dpos, dfv, derr))) break;
         int herr = 0;
         if (hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||

@@ -236,9 +236,7 @@ template <typename T>
 int launch_bcsr_sweep(Ctx *c, const Schedule &s, bool upper, int N, int bnl, int bnw, const int *brptr,
                       const int *bcind, const T *bval, const T *x, T *y, bool *done);
 template <typename T>
-int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *cind, const int *dpos, T *val,
-                int *derr);
-int launch_find_diag(Ctx *c, int N, const int *rptr, const int *cind, int *dpos);
+int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *cind, int *dpos, T *val, int *derr);
 // d = diag(U) (from U's inverted diagonal, first in each row), e = 2 d - diag(A), FP32
 int launch_ic_upper(Ctx *c, int lnnz, const int *umap, const int *lcol, const double *f, const int *dpos,
                     const double *l, double *u);

@@ -912,7 +912,7 @@ __global__ __launch_bounds__((kIluThreads<BS, G>)) void k_ilu0_group(
 }
 
 // k_ilu0, for what the kernel above does not hold (blocks that do not divide 64, workgroups
-// of more than kIluLdsBytes of entries): one wave per schedule block; the block's rows are
+// of more than kIluLdsBytes of entries, rows whose columns do not ascend): one wave per schedule block; the block's rows are
 // factored in order.  A row of up
 // to 64*R entries lives in registers (lane q holds entries q, q+64, ...; R = 4, 16 or 64
 // by the longest row of the factor, so rows of up to 4096 entries).  For every
@@ -1028,6 +1028,31 @@ __global__ __launch_bounds__(kBlock) void k_max_row_len(int N, const int *__rest
 __global__ void k_zero_i(int n, int *p) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
 }
+// dpos[i]: the place of row i's diagonal entry, or -1; *unordered becomes 1 if the columns of a
+// row do not strictly ascend.
+__global__ __launch_bounds__(kBlock) void k_find_diag(int N, const int *__restrict__ rptr,
+                                                      const int *__restrict__ cind, int *__restrict__ dpos,
+                                                      int *unordered) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= N) return;
+    int p = -1, prev = -1;
+    bool bad = false;
+    const int e = rptr[i + 1];
+    for (int j0 = rptr[i]; j0 < e; j0 += 8) {  // eight independent loads at a time
+        int c[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) c[u] = j0 + u < e ? cind[j0 + u] : -1;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (j0 + u < e) {
+                if (c[u] == i && p < 0) p = j0 + u;
+                bad |= c[u] <= prev;
+                prev = c[u];
+            }
+    }
+    dpos[i] = p;
+    if (bad) *unordered = 1;
+}
 constexpr int kIluLdsBytes = 64 * 1024;
 template <typename T, int BS, int G>
 static int ilu0_group_levels(Ctx *c, const Schedule &s, const int *rptr, const int *cind, const int *dpos, T *val,
@@ -1061,16 +1086,17 @@ static int ilu0_levels(Ctx *c, const Schedule &s, const int *rptr, const int *ci
     return SENK_OK;
 }
 template <typename T>
-int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *cind, const int *dpos, T *val,
-                int *derr) {
+int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *cind, int *dpos, T *val, int *derr) {
     if (N <= 0) return SENK_OK;
     int *dmax = reinterpret_cast<int *>(c->dscalars), *h = c->hpinned_i;
-    k_zero_i<<<1, 64, 0, c->stream>>>(2, dmax);
+    k_zero_i<<<1, 64, 0, c->stream>>>(3, dmax);
+    SENK_LAUNCH_CHECK();
+    k_find_diag<<<(N + kBlock - 1) / kBlock, kBlock, 0, c->stream>>>(N, rptr, cind, dpos, dmax + 2);
     SENK_LAUNCH_CHECK();
     k_max_row_len<<<std::max(1, std::min((N + kBlock - 1) / kBlock, kMaxRowLenGrid)), kBlock, 0, c->stream>>>(N, rptr,
                                                                                                            dmax);
     SENK_LAUNCH_CHECK();
-    SENK_HIP(hipMemcpyAsync(h, dmax, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    SENK_HIP(hipMemcpyAsync(h, dmax, 3 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     SENK_HIP(hipStreamSynchronize(c->stream));
     const int maxlen = h[0];
     bool done = false;
@@ -1081,7 +1107,7 @@ int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *ci
                  ? ilu0_group_levels<T, B, 4>(c, s, rptr, cind, dpos, val, derr, maxlen, h[1], &done)         \
                  : ilu0_group_levels<T, B, 16>(c, s, rptr, cind, dpos, val, derr, maxlen, h[1], &done);       \
         break;
-    switch (s.bsize) {
+    switch (h[2] ? 0 : s.bsize) {  // it looks columns up among a row's own, which must ascend
         SENK_ILU_GROUP(1)
         SENK_ILU_GROUP(2)
         SENK_ILU_GROUP(4)
@@ -1098,26 +1124,8 @@ int launch_ilu0(Ctx *c, const Schedule &s, int N, const int *rptr, const int *ci
     if (maxlen <= 64 * 16) return ilu0_levels<T, 16>(c, s, rptr, cind, dpos, val, derr);
     return ilu0_levels<T, 64>(c, s, rptr, cind, dpos, val, derr);
 }
-template int launch_ilu0<double>(Ctx *, const Schedule &, int, const int *, const int *, const int *, double *,
-                                 int *);
-template int launch_ilu0<float>(Ctx *, const Schedule &, int, const int *, const int *, const int *, float *,
-                                int *);
-
-__global__ __launch_bounds__(kBlock) void k_find_diag(int N, const int *__restrict__ rptr,
-                                                      const int *__restrict__ cind, int *__restrict__ dpos) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= N) return;
-    int p = -1;
-    for (int j = rptr[i]; j < rptr[i + 1]; j++)
-        if (cind[j] == i) { p = j; break; }
-    dpos[i] = p;
-}
-int launch_find_diag(Ctx *c, int N, const int *rptr, const int *cind, int *dpos) {
-    if (N <= 0) return SENK_OK;
-    k_find_diag<<<(N + kBlock - 1) / kBlock, kBlock, 0, c->stream>>>(N, rptr, cind, dpos);
-    SENK_LAUNCH_CHECK();
-    return SENK_OK;
-}
+template int launch_ilu0<double>(Ctx *, const Schedule &, int, const int *, const int *, int *, double *, int *);
+template int launch_ilu0<float>(Ctx *, const Schedule &, int, const int *, const int *, int *, float *, int *);
 
 // D-ILU vectors: d = diag(U) from U's inverted diagonal (first entry of each row),
 // e = 2 d - diag(A), both rounded to FP32

@@ -67,3 +67,39 @@ def test_zero_pivot_inside_and_outside_the_block(ctx, where):
     d = [ctx.array(np.array(t, dt)) for t, dt in ((val, np.float64), (cind, np.int32), (rptr, np.int32))]
     cptr = np.array([0, 1, 2], np.int32)
     assert S.lib().senk_ilu0_f64(ctx.h, *(t.p for t in d), N, O.P(cptr), 2, bs, None, None) == 3
+
+
+def _elimination(val, cind, rptr, N):
+    """ILU(0) by columns, whatever the order of a row's later entries: every entry gets its updates
+    in increasing pivot column."""
+    v, at = val.copy(), [dict(zip(cind[rptr[i]:rptr[i + 1]].tolist(), range(rptr[i], rptr[i + 1]))) for i in range(N)]
+    for i in range(N):
+        for k in sorted(c for c in at[i] if c < i):
+            l = v[at[i][k]] / v[at[k][k]]
+            v[at[i][k]] = l
+            for c, q in at[i].items():
+                if c > k and c in at[k]:
+                    v[q] -= l * v[at[k][c]]
+    return v
+
+
+@pytest.mark.parametrize("order", ["ascending", "shuffled"])
+def test_rows_whose_later_entries_are_in_any_order(ctx, order):
+    """Entries beyond the diagonal out of order, in rows that no other row eliminates with."""
+    rng, h = np.random.default_rng(3), 48
+    N, rows = 2 * h, []
+    for i in range(N):
+        up = np.arange(i + 1, N)
+        up = np.sort(rng.choice(up, min(len(up), 14), replace=False))
+        if i >= h and order == "shuffled":
+            up = rng.permutation(up)
+        low = np.sort(rng.choice(min(i, h), min(i, h, 9), replace=False)) if i else np.zeros(0, int)
+        rows.append(np.concatenate([low, [i], up]))
+    rptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    cind = np.concatenate(rows).astype(np.int32)
+    val = rng.uniform(-1, 1, len(cind))
+    for i in range(N):
+        val[rptr[i] + np.flatnonzero(rows[i] == i)[0]] = 20.0
+    d = [ctx.array(t) for t in (val, cind, rptr)]
+    S.call("senk_ilu0_f64", ctx.h, *(t.p for t in d), N, None, 0, 1, O.P(rptr), O.P(cind))
+    assert np.array_equal(d[0].download(), _elimination(val, cind, rptr, N))
