@@ -34,8 +34,7 @@ def test_colored_bitwise(ctx, bsize, gen, dt):
     assert np.array_equal(f, fo)
 
 
-# dependency levels (lists of rows); 16 and 17 entries a row, and rows whose workgroup exceeds
-# the LDS limit (the wave-per-block kernel)
+# dependency levels (lists of rows), up to 16 entries a row, 17, and up to 225
 @pytest.mark.parametrize("width", [7, 16, 17, 90, 400])
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_levels_of_banded_rows_bitwise(ctx, width, dt):
@@ -48,6 +47,37 @@ def test_levels_of_banded_rows_bitwise(ctx, width, dt):
     for i in range(N):
         val[rptr[i] + np.searchsorted(rows[i], i)] = 2.0 + len(rows[i])
     f, fo = _factor(ctx, val, cind, rptr, N, dt)
+    assert np.array_equal(f, fo)
+
+
+def _rows_of(N, width, seed):
+    """Rows of exactly `width` ascending columns, near the diagonal, which is among them."""
+    rng, out = np.random.default_rng(seed), []
+    for i in range(N):
+        lo = min(max(0, i - width), N - 2 * width)
+        c = rng.choice(np.setdiff1d(np.arange(lo, lo + 2 * width), [i]), width - 1, replace=False)
+        out.append(np.sort(np.append(c, i)))
+    rptr = (np.arange(N + 1) * width).astype(np.int32)
+    cind = np.concatenate(out).astype(np.int32)
+    val = rng.uniform(-1, 1, len(cind))
+    val[cind == np.repeat(np.arange(N), width)] = 2.0 + width
+    return rptr, cind, val
+
+
+# The grouped kernel holds up to 64 KB of entries (12 bytes in FP64, 8 in FP32) per workgroup of
+# 16 rows, or of 64 in blocks of 64: the longest rows it takes and the shortest it hands on.
+@pytest.mark.parametrize("bsize,dt,width", [(1, np.float64, 341), (1, np.float64, 342), (1, np.float32, 512),
+                                            (1, np.float32, 513), (8, np.float64, 341), (8, np.float64, 342),
+                                            (64, np.float64, 85), (64, np.float64, 86), (64, np.float32, 128),
+                                            (64, np.float32, 129)])
+def test_rows_around_the_lds_limit_bitwise(ctx, bsize, dt, width):
+    N = 1152
+    rptr, cind, val = _rows_of(N, width, width)
+    if bsize == 1:  # dependency levels
+        f, fo = _factor(ctx, val, cind, rptr, N, dt)
+    else:
+        sy = abmc_system(rptr, cind, val, bsize)
+        f, fo = _factor(ctx, sy["val"], sy["cind"], sy["rptr"], N, dt, sy["cptr"], sy["nc"], bsize)
     assert np.array_equal(f, fo)
 
 
