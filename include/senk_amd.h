@@ -133,7 +133,20 @@ int senk_spmv_sellcs_f32(senk_ctx ctx, const senk_sellcs *dev, const float *dx, 
 /* SptrsvCsr_l / SptrsvCsr_u, ABMC form      senk_sparse.hpp:250-315.
  * cptr (host, cnum+1 entries) counts blocks of bsize rows.  L holds the strict lower
  * part; U holds the inverted diagonal first in each row ("L-DU", invDiag).  x may
- * alias y for the U solve. */
+ * alias y for the U solve.
+ *
+ * These solves, the planned and the block ones below run in one launch per triangle in which
+ * rows wait for the rows they read.  Two consequences for the caller:
+ *  - the colors (cptr) must be valid for the factor: no row may read a row of another block of
+ *    its own color or of a later one.  That cannot be checked here (the pattern is on the
+ *    device); such a solve waits in vain until its polls run out (seconds, see
+ *    senk_ctx_set_trsv_polls), its result is invalid, and the next call that hands a result to
+ *    the host returns SENK_ERR_TIMEOUT;
+ *  - the context keeps two vectors of the longest such solve so far (N values, a plan's rows
+ *    padded to whole waves).  The first solve and every longer one wait for the context's
+ *    stream and allocate them; senk_ctx_destroy gives them back.  Without memory for them, and
+ *    for schedules the launch does not take (blocks that do not divide 64 rows in the CSR form,
+ *    more than 256 colors, colors that stop short of N), a launch per level runs instead. */
 int senk_sptrsv_csr_l_abmc_f64(senk_ctx ctx, const double *dval, const int *dcind, const int *drptr,
                                const double *dx, double *dy, int N, const int *cptr, int cnum, int bsize);
 int senk_sptrsv_csr_u_abmc_f64(senk_ctx ctx, const double *dval, const int *dcind, const int *drptr,
@@ -155,7 +168,8 @@ int senk_sptrsv_csr_u_amc_f32(senk_ctx ctx, const float *dval, const int *dcind,
 /* Sequential and block-Jacobi forms (senk_sparse.hpp:132-167, 328-379) need the
  * dependency levels of the factor, computed once on the host from its pattern:
  * rows of one level are independent, and every row's sum keeps the reference's CSR
- * order, so the result equals the sequential solve. */
+ * order, so the result equals the sequential solve.  A plan holds three integers a row on the
+ * device (the levels, the order of the solve and each row's place in it). */
 typedef struct senk_trsv_plan_s *senk_trsv_plan;
 /* upper = 0 for L (strict lower), 1 for U (diagonal first).  rptr/cind are host arrays. */
 int senk_trsv_plan_create(senk_ctx ctx, const int *rptr, const int *cind, int N, int upper,
