@@ -140,6 +140,7 @@ struct TriLayout {
     int *next = nullptr;         // bsize 64 only: per slot external count
     int *scol = nullptr;         // n_ext external columns
     bool cols_filled = false;
+    float line_lanes64 = 0, line_lanes32 = 0;  // lanes of a gather per 128-byte line (0: not counted)
     double *ve64 = nullptr, *vi64 = nullptr, *d64 = nullptr;  // values; d = inverted diagonal (U)
     float *ve32 = nullptr, *vi32 = nullptr, *d32 = nullptr;
     unsigned *sync = nullptr;    // sweep time-out flag, spares

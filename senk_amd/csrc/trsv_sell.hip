@@ -151,7 +151,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill(int nslices, const int4 *__
                                                      const typename RowWord<BS>::W *__restrict__ rw,
                                                      const int *__restrict__ next, int *__restrict__ scol,
                                                      V *__restrict__ ve, V *__restrict__ vi,
-                                                     DiagT<V> *__restrict__ dinv, signed char *__restrict__ sx) {
+                                                     DiagT<V> *__restrict__ dinv, signed char *__restrict__ sx,
+                                                     unsigned *lines) {
     const int w = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
     if (w >= nslices) return;
     const int4 si = sinfo[w];
@@ -177,17 +178,29 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill(int nslices, const int4 *__
         else return (V)v;
     };
     int pos = si.x;
+    unsigned nl[2] = {0, 0};
     for (int k = 0;; k++) {
         const unsigned long long b = __ballot(k < ne);
         if (!b) break;
+        int c = 0;
         if (k < ne) {
             const int j = UPPER ? e - 1 - k : s + k;
             const int p = pos + lanes_below(b);
-            if (scol) scol[p] = cind[j];
+            c = cind[j];
+            if (scol) scol[p] = c;
             ve[p] = enc(val[j]);
         }
         pos += __popcll(b);
+        if (lines) {  // distinct 128-byte lines that this gather touches, FP64 and FP32
+#pragma unroll
+            for (int f = 0; f < 2; f++)
+                for (unsigned long long left = b; left; nl[f]++) {
+                    const int l = __builtin_amdgcn_readlane(c >> (4 + f), __ffsll((long long)left) - 1);
+                    left &= ~__ballot(c >> (4 + f) == l);
+                }
+        }
     }
+    if (lines && (threadIdx.x & 63) < 2) atomicAdd(lines + (threadIdx.x & 63), (threadIdx.x & 63) ? nl[1] : nl[0]);
     int q = UPPER ? e - 1 - ne : s + ne;
     int ipos = si.y;
     for (int i = 0; i < BS; i++) {
@@ -204,7 +217,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_fill(int nslices, const int4 *__
 }
 
 // Sweep words (unsigned, device): the time-out flag and the ticket counter of mode 2.
-constexpr int kSweepErr = 0, kSweepTicket = 1, kSweepWords = 32;
+// kSweepLines: two counts of the layout's construction (tri_lines_wanted).
+constexpr int kSweepErr = 0, kSweepTicket = 1, kSweepLines = 8, kSweepWords = 32;
 // workgroup size (waves = slices per ticket) of the per-XCD ticket streams: 8-wave
 // workgroups measured best (FP32 application at 128^3, connect blocks of 8, with one
 // ticket counter per XCD: 71.5 us, 77.4 with 16 waves, 73.0 with 4)
@@ -344,9 +358,7 @@ __device__ __forceinline__ void solve_slice_body(const SliceHead<V, BS> &h, cons
             // between polls: ALL, where launch_xticket still takes it) the polls themselves slowed
             // the rows waited for down: FP32 application, 7-point 96^3 connect blocks of 8, 75.8 ->
             // 56.3 us; FP64, 27-point 71^3 blocks of 16, 131.8 -> 108.7 us, unstructured 300,000
-            // rows 550 -> 485 us.  Where the rows of a level end together the second read is a
-            // round trip more: 27-point systems of 32^3 to 48^3 in 8 colors of whole lines (simple
-            // blocks of 8) lose 3%, those whose lines the blocks cut gain 8-13%.
+            // rows 550 -> 485 us.
             if constexpr (ALL) {
                 bool pend = false;
 #pragma unroll
@@ -644,14 +656,14 @@ int count_rows(Ctx *c, const Schedule &s, const TriLayout &L, const int *rptr, c
 
 template <typename S, typename V, int BS>
 int fill_rows(Ctx *c, const Schedule &s, const TriLayout &L, const int *rptr, const int *cind, const S *val, int *scol,
-              V *ve, V *vi, DiagT<V> *dinv, signed char *sx) {
+              V *ve, V *vi, DiagT<V> *dinv, signed char *sx, unsigned *lines) {
     using W = typename RowWord<BS>::W;
     if (L.upper)
         k_tri_fill<S, V, BS, true><<<waves_grid(L.nslices), kBlock, 0, c->stream>>>(
-            L.nslices, L.sinfo, s.dblk, rptr, cind, val, (const W *)L.rw, L.next, scol, ve, vi, dinv, sx);
+            L.nslices, L.sinfo, s.dblk, rptr, cind, val, (const W *)L.rw, L.next, scol, ve, vi, dinv, sx, lines);
     else
         k_tri_fill<S, V, BS, false><<<waves_grid(L.nslices), kBlock, 0, c->stream>>>(
-            L.nslices, L.sinfo, s.dblk, rptr, cind, val, (const W *)L.rw, L.next, scol, ve, vi, dinv, sx);
+            L.nslices, L.sinfo, s.dblk, rptr, cind, val, (const W *)L.rw, L.next, scol, ve, vi, dinv, sx, lines);
     SENK_LAUNCH_CHECK();
     return SENK_OK;
 }
@@ -759,8 +771,19 @@ int launch_xticket(Ctx *c, const Schedule &s, TriLayout &L, const V *ve, const V
     // 17.6 / 16.8, 80^3 (15.6) 19.2 / 17.6, 128^3 (64) 63.6 / 60.5; blocks of 8, 1000 x 800 (24)
     // equal; FP32 27-point simple blocks of 16, 96^3 (6.8) 64.7 / 67.5, 112^3 (10.7) 91.0 / 88.8,
     // 128^3 (16) 127.8 / 119.0.  The other kernels keep their waves and run the same either way.
-    const bool all = (ch4 || (std::is_same<T, float>::value && pipe)) && L.max_ext <= 32 &&
-                     (long long)L.nslices > (ch4 ? 13LL : 10LL) * c->num_cus * L.nsteps;
+    //
+    // So do rows of more than 8 entries in 8 levels or more where the lanes of a gather share
+    // their lines (blocks that are runs of whole lines of the grid): polling all of them is then a
+    // few lines, and the one-row wait only adds its second read.  One row / all, us, with the lanes
+    // per 128-byte line: 27-point FP64, 48^3 simple blocks of 8 (8.1) 33.5 / 32.5, 32^3 (8.5) 33.3 /
+    // 31.5, 64^3 connect blocks of 8 (6.8) 41.1 / 44.9, 36^3 simple blocks of 8 (4.7) 35.9 / 38.8; FP32
+    // 48^3 (14.2) 28.9 / 28.2, 64^3 connect (12.5) 33.6 / 37.0.  In 4 levels, 16^3 blocks of 16
+    // (11.3) 21.4 / 23.6.
+    const bool large = (ch4 || (std::is_same<T, float>::value && pipe)) &&
+                       (long long)L.nslices > (ch4 ? 13LL : 10LL) * c->num_cus * L.nsteps;
+    const bool shared = !ch4 && pipe && L.nsteps >= 8 &&
+                        (std::is_same<T, double>::value ? L.line_lanes64 >= 7.5f : L.line_lanes32 >= 13.f);
+    const bool all = L.max_ext <= 32 && (large || shared);
     // 32-bit byte offsets where every array the sweep indexes fits them (elements of at most
     // 8 bytes; the slice descriptors, 16 bytes each, number at most a 64th of the slots)
     const long long most = std::max({(long long)L.n, L.n_ext, L.n_int, (long long)L.nslices * 64});
@@ -780,7 +803,8 @@ int launch_xticket(Ctx *c, const Schedule &s, TriLayout &L, const V *ve, const V
     // of 8; the 27-point system, rows of 17-32, loses with them: FP64 315 against 246 us)
     if (all) {
         if constexpr (std::is_same<V, double>::value) {
-            if (pipe) SENK_XT_LAUNCH(4, true, true);
+            if (!ch4) SENK_XT_LAUNCH(8, true, true);
+            else if (pipe) SENK_XT_LAUNCH(4, true, true);
             else SENK_XT_LAUNCH(4, false, true);
         } else {
             SENK_XT_LAUNCH(8, true, true);
@@ -982,6 +1006,21 @@ int tri_layout_build(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
     return fail(SENK_OK);
 }
 
+// Whether the wait of this layout's sweeps depends on how many lanes of a gather share a line
+// (launch_xticket), which is counted as the columns are filled in.
+static bool tri_lines_wanted(const TriLayout &L) {
+    return !L.cols_filled && L.nsteps >= 8 && L.max_ext > 8 && L.max_ext <= 32;
+}
+static int tri_lines_done(Ctx *c, TriLayout *L, const unsigned *lines) {
+    if (!lines) return SENK_OK;
+    unsigned h[2] = {0, 0};
+    SENK_HIP(hipMemcpyAsync(h, lines, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+    SENK_HIP(hipStreamSynchronize(c->stream));
+    L->line_lanes64 = h[0] ? (float)L->n_ext / (float)h[0] : 0.f;
+    L->line_lanes32 = h[1] ? (float)L->n_ext / (float)h[1] : 0.f;
+    return SENK_OK;
+}
+
 template <typename T>
 int tri_layout_fill(Ctx *c, const Schedule &s, TriLayout *L, const int *rptr, const int *cind, const T *val) {
     if (L->nslices == 0) return SENK_OK;
@@ -1000,10 +1039,12 @@ int tri_layout_fill(Ctx *c, const Schedule &s, TriLayout *L, const int *rptr, co
         SENK_TRY(fill_sentinel<T>(c, L->n, (T *)*mid));
     }
     int *scol = L->cols_filled ? nullptr : L->scol;
+    unsigned *lines = tri_lines_wanted(*L) ? L->sync + kSweepLines : nullptr;
     auto run = [&]() -> int {
-        SENK_BS_DISPATCH(L->bsize, (fill_rows<T, T, B>(c, s, *L, rptr, cind, val, scol, *ve, *vi, *dv, nullptr)))
+        SENK_BS_DISPATCH(L->bsize, (fill_rows<T, T, B>(c, s, *L, rptr, cind, val, scol, *ve, *vi, *dv, nullptr, lines)))
     };
     SENK_TRY(run());
+    SENK_TRY(tri_lines_done(c, L, lines));
     L->cols_filled = true;
     return SENK_OK;
 }
@@ -1021,11 +1062,13 @@ int tri_layout_fill_f16(Ctx *c, const Schedule &s, TriLayout *L, const int *rptr
         SENK_TRY(fill_sentinel<float>(c, L->n, (float *)L->mid32));
     }
     int *scol = L->cols_filled ? nullptr : L->scol;
+    unsigned *lines = tri_lines_wanted(*L) ? L->sync + kSweepLines : nullptr;
     auto run = [&]() -> int {
         SENK_BS_DISPATCH(L->bsize, (fill_rows<double, __half, B>(c, s, *L, rptr, cind, val, scol, (__half *)L->ve16,
-                                                                 (__half *)L->vi16, L->d16, L->sx16)))
+                                                                 (__half *)L->vi16, L->d16, L->sx16, lines)))
     };
     SENK_TRY(run());
+    SENK_TRY(tri_lines_done(c, L, lines));
     L->cols_filled = true;
     return SENK_OK;
 }

@@ -151,6 +151,15 @@ def test_layout_abmc_unstructured_long_rows(ctx):
     _check(ctx, sy, S.SENK_ILU0, 0, 16, colors=True)
 
 
+# eight colors of whole grid lines: the lanes of a gather share lines, and a wait polls all rows;
+# blocks of 16 cut the lines of 20 (6 colors), and one row is polled
+@pytest.mark.parametrize("n,bsize", [(16, 4), (16, 8), (24, 8), (20, 16)])
+def test_layout_gathers_that_share_lines(ctx, n, bsize):
+    rptr, cind, val = S.gen_convdiff27(n, 10.0)
+    sy = abmc_system(rptr, cind, val, bsize, "simple")
+    _check(ctx, sy, S.SENK_ILU0, 0, bsize, True)
+
+
 # levels of 3400 slices, above the lines from which a wait polls all of its rows: FP64 rows of one
 # round of gathers (4) and of two (6), FP32 rows of two (12)
 @pytest.mark.parametrize("k,bsize", [(4, 8), (6, 1), (12, 8)])
