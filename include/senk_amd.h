@@ -508,7 +508,8 @@ int senk_prec_apply_f16(senk_prec M, const float *dx, float *dy);
  * level, so a wait is only on workgroups handed out earlier); the default, which -1
  * restores.  Results are
  * bit-identical in every mode.  Applications of one preconditioner must not overlap (one
- * stream). */
+ * stream).  Where preconditioners of several contexts or processes are applied at the same
+ * time on one device, mode 2 (or 0) is the one that cannot hold another up. */
 int senk_prec_set_trsv_mode(senk_prec M, int mode);
 /* Split form of the mixed forms' inner BiCGStab (no reference counterpart; the
  * reference's BiCGStab is right-preconditioned, senk_bicgstab.hpp:129-161).  When the

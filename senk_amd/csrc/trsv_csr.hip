@@ -409,7 +409,7 @@ __global__ __launch_bounds__(64) void k_csr_rows(int waves, int xcds, const int 
 // broadcast in the wave; the lane's next in-part blocks wait in LDS, requested before the
 // first wait, one block read ahead of its step (in registers instead of LDS the queue spills:
 // 181-604 us).  Bound by the levels' chain (publish, poll, in-part steps).  Elasticity 45^3,
-// blocks of 48, 11 colors, L + U in FP64: 155 us; one lane per schedule block walking its rows,
+// blocks of 48, 11 colors, L + U in FP64: 150 us; one lane per schedule block walking its rows,
 // one launch per color (518 lanes in flight), 3187 us.
 template <typename T, int BNL, int BNW, bool UPPER>
 __global__ __launch_bounds__(64 * kCsrWaves) void k_bcsr_sweep(
