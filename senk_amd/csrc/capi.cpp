@@ -68,6 +68,10 @@ static int arena_get(DevBuf &a, size_t bytes, void **out) {
 int ctx_sweep_check(Ctx *c) {
     if (!c->sweep_err || !__atomic_load_n(c->sweep_err, __ATOMIC_ACQUIRE)) return SENK_OK;
     __atomic_store_n(c->sweep_err, 0u, __ATOMIC_RELEASE);
+    // the next solve starts from filled vectors and a counter in step with the host's count
+    c->sweep.spoiled();
+    (void)hipMemsetAsync(c->sweep_ticket, 0, sizeof(unsigned), c->stream);
+    c->sweep_base = 0;
     record_error("a single-launch triangular solve gave up a wait");
     return SENK_ERR_TIMEOUT;
 }

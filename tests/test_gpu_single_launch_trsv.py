@@ -261,13 +261,21 @@ def _chain(ctx, n, dt=np.float64):
     return run, dy, y
 
 
+@pytest.mark.parametrize("tickets", [0, 1])
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
-def test_poll_limit(ctx, dt):
+def test_poll_limit(ctx, dt, tickets):
     run, dy, y = _chain(ctx, 500, dt)
-    assert _gives_up(ctx, run) == 11
-    assert S.lib().senk_ctx_synchronize(ctx.h) == 0
-    run()
-    assert np.array_equal(dy.download(), y)
+    assert S.lib().senk_ctx_set_trsv_tickets(ctx.h, tickets) == 0
+    try:
+        for _ in range(2):
+            assert _gives_up(ctx, run) == 11
+            assert S.lib().senk_ctx_synchronize(ctx.h) == 0
+            run()
+            assert np.array_equal(dy.download(), y)
+            run()
+            assert np.array_equal(dy.download(), y)
+    finally:
+        S.lib().senk_ctx_set_trsv_tickets(ctx.h, -1)
     assert S.lib().senk_ctx_set_trsv_polls(ctx.h, -1) == 1
 
 
