@@ -325,12 +325,13 @@ int senk_ctx_create(int device, senk_ctx *out) {
     c.device = device;
     SENK_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
     SENK_HIP(hipMalloc(&c.red_partials, sizeof(double) * kRedSlots * kRedMaxK * kRedMaxBlocks));
-    SENK_HIP(hipMalloc(&c.dscalars, sizeof(double) * 64));
+    SENK_HIP(hipMalloc(&c.dscalars, sizeof(double) * (64 + 16)));
     SENK_HIP(hipHostMalloc((void **)&c.hpinned, sizeof(double) * 64, hipHostMallocDefault));
     SENK_HIP(hipHostMalloc((void **)&c.hpinned_i, sizeof(int) * 64, hipHostMallocDefault));
     SENK_HIP(hipHostMalloc((void **)&c.sweep_err, 64, hipHostMallocCoherent));
     *c.sweep_err = 0;
-    SENK_HIP(hipMalloc(&c.sweep_ticket, sizeof(unsigned)));
+    // the ticket counter on a line of its own behind the scalars
+    c.sweep_ticket = reinterpret_cast<unsigned *>(c.dscalars + 64);
     SENK_HIP(hipMemset(c.sweep_ticket, 0, sizeof(unsigned)));
     SENK_HIP(hipHostGetDevicePointer((void **)&c.sweep_err_d, c.sweep_err, 0));
     hipDeviceProp_t prop;
@@ -367,7 +368,6 @@ int senk_ctx_destroy(senk_ctx ctx) {
     (void)hipFree(c.dscalars);
     for (SweepVec &v : c.sweep.v)
         if (v.p) (void)hipFree(v.p);
-    (void)hipFree(c.sweep_ticket);
     (void)hipHostFree(c.sweep_err);
     (void)hipHostFree(c.hpinned);
     (void)hipHostFree(c.hpinned_i);
