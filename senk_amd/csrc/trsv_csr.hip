@@ -795,9 +795,9 @@ int launch_csr_sweep(Ctx *c, const Schedule &s, bool upper, int N, const int *rp
         SweepLaunch sl(c);
         // rounds of 4 where no row has more entries, else of 16: a second round costs its own
         // chain of dependent loads after the last row of the first is there
-#define SENK_CSR_ROWS(UP, CH)                                                                                      \
-    k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.seq_waves, s.streams, s.dseq, s.dpos, rptr, cind, val, x, y, z, reset, \
-                                                      UP ? nullptr : in_scale, sl.wt, stop)
+#define SENK_CSR_ROWS(UP, CH)                                                                                     \
+    k_csr_rows<T, UP, CH><<<grid, 64, 0, c->stream>>>(s.seq_waves, s.streams, s.dseq, s.dpos, rptr, cind, val, x, \
+                                                      y, z, reset, UP ? nullptr : in_scale, sl.wt, stop)
         if (upper && s.max_ext <= 4) SENK_CSR_ROWS(true, 4);
         else if (upper) SENK_CSR_ROWS(true, 16);
         else if (s.max_ext <= 4) SENK_CSR_ROWS(false, 4);
@@ -846,8 +846,9 @@ template int launch_csr_sweep<float>(Ctx *, const Schedule &, bool, int, const i
                                      const float *, float *, const double *, const int *, bool *);
 
 template <typename T, int BNL, int BNW>
-static void bcsr_sweep(Ctx *c, const SweepWait &wt, const SweepLevels &lv, int tickets, const Schedule &s, bool upper, int part, int bpw,
-                       const int *brptr, const int *bcind, const T *bval, const T *x, T *y, T *z, T *reset) {
+static void bcsr_sweep(Ctx *c, const SweepWait &wt, const SweepLevels &lv, int tickets, const Schedule &s,
+                       bool upper, int part, int bpw, const int *brptr, const int *bcind, const T *bval, const T *x,
+                       T *y, T *z, T *reset) {
     const int grid = kXcds * tickets;
     if (upper)
         k_bcsr_sweep<T, BNL, BNW, true><<<grid, 64 * kCsrWaves, 0, c->stream>>>(
